@@ -43,7 +43,9 @@ extern "C" {
 /* IEEE binary16 value held as its raw bits (quantized-KV scales). */
 typedef uint16_t f16_storage_t;
 
-/* ABI version; bumped when entry points are added or their signatures change. */
+/* ABI version; bumped when an entry point's signature or layout changes.
+ * Entry points may be added within a version: a binding looks up every one it
+ * calls when it loads the library. */
 int mk_abi_version(void);
 
 /* ---------------------------------------------------------------- q4/q8 pack / dequant */
@@ -251,6 +253,12 @@ int mk_qkv_rope_paged_update_quant(const void* qkv, const float* cos_t, const fl
  * quantizer of :146-175 (correctly rounded fp32 divide, round half to even). */
 int mk_quantize_kv(const void* src, uint8_t* codes, f16_storage_t* scales, int64_t rows, int64_t D,
                    int64_t group_size, int bits, int dtype, void* stream);
+
+/* dequantize_kv_pages -- ops/paged_quantized_kv_ops.py:295-341 for one of K
+ * or V: codes and scales as mk_quantize_kv lays them out -> out [rows, D]
+ * fp16, (code - 128|8) * |scale| in fp32 and rounded once. */
+int mk_dequantize_kv(const uint8_t* codes, const f16_storage_t* scales, void* out, int64_t rows, int64_t D,
+                     int64_t group_size, int bits, void* stream);
 
 /* ---------------------------------------------------------------- paged decode attention */
 

@@ -308,6 +308,113 @@ __global__ void quantize_kv_rows_kernel(const T* __restrict__ src, uint8_t* __re
   }
 }
 
+// The same quantizer for rows of whole groups of 8 << lgl values (lgl <= 6):
+// a thread takes 8 consecutive values (one 16-byte load), the 1 << lgl lanes
+// of a group share its absmax by shuffles, and each thread stores its 8 codes
+// in one piece.  Rows hold whole groups, so neither rows nor groups matter to
+// the indexing: value chunk i belongs to group i >> lgl.  Bound by memory:
+// the row-per-thread kernel above reads 2 bytes per lane at a stride of a
+// row (K or V of 4 x 8192 positions, 8 heads of 128, q8:
+// 570 us a tensor there, 27.9 us here for its 103 MB).
+template <typename T, int BITS>
+__global__ __launch_bounds__(256) void quantize_kv_vec_kernel(const T* __restrict__ src, uint8_t* __restrict__ codes,
+                                                              uint16_t* __restrict__ scales, int64_t chunks,
+                                                              int lgl) {
+  const int64_t i0 = blockIdx.x * (int64_t)256 + threadIdx.x;
+  const bool live = i0 < chunks;  // whole groups are live or not: chunks is a multiple of 1 << lgl
+  const int64_t i = live ? i0 : 0;
+  const float qmax = BITS == 8 ? 127.0f : 7.0f;
+  const float qoff = BITS == 8 ? 128.0f : 8.0f;
+  const u32x4 raw = ldg128_stream(src + 8 * i);
+  float v[8];
+  float amax = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    v[e] = to_f32(bitcast<T>((uint16_t)(raw[e >> 1] >> (16 * (e & 1)))));
+    amax = fmaxf(amax, fabsf(v[e]));
+  }
+  for (int o = 0; o < lgl; ++o) amax = fmaxf(amax, __shfl_xor(amax, 1 << o, MK_WAVE));
+  amax = fmaxf(amax, 1e-8f);
+  const float scale = amax / qmax;  // correctly rounded fp32 division
+  uint32_t c[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float qv = rintf(v[e] / scale);
+    qv = fminf(fmaxf(qv, -qmax), qmax);
+    c[e] = (uint32_t)(int)(qv + qoff);
+  }
+  if (!live) return;
+  if ((i & ((1 << lgl) - 1)) == 0) scales[i >> lgl] = bitcast<uint16_t>((f16)scale);
+  if constexpr (BITS == 8) {
+    const u32x2 o = {c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24),
+                     c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24)};
+    *reinterpret_cast<u32x2*>(codes + 8 * i) = o;
+  } else {
+    uint32_t o = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o |= c[e] << (4 * e);
+    *reinterpret_cast<uint32_t*>(codes + 4 * i) = o;
+  }
+}
+
+// Codes back to fp16 values, (code - 128|8) * |scale| in fp32 and rounded
+// once (ops/paged_quantized_kv_ops.py:156-186, 295-341): 8 consecutive values
+// of one group (1 << lgl chunks) per thread, one 16-byte store.  Bound by
+// memory: 16.6 us for the 103 MB above (6.2 TB/s, part of it from the
+// Infinity Cache) against 270 us for the five tensor ops that it replaces.
+template <int BITS>
+__global__ __launch_bounds__(256) void dequantize_kv_vec_kernel(const uint8_t* __restrict__ codes,
+                                                                const uint16_t* __restrict__ scales,
+                                                                f16* __restrict__ out, int64_t chunks, int lgl) {
+  const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (i >= chunks) return;
+  const float s = fabsf((float)bitcast<f16>(scales[i >> lgl]));
+  u32x2 q;
+  if constexpr (BITS == 8) q = ldg64_stream(codes + 8 * i);
+  else q[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(codes + 4 * i));
+  u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    uint32_t h[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t c = BITS == 8 ? (q[(e + j) >> 2] >> (8 * ((e + j) & 3))) & 255u : (q[0] >> (4 * (e + j))) & 15u;
+      h[j] = bitcast<uint16_t>((f16)(((float)c - (BITS == 8 ? 128.0f : 8.0f)) * s));
+    }
+    o[e >> 1] = h[0] | (h[1] << 16);
+  }
+  *reinterpret_cast<u32x4*>(out + 8 * i) = o;
+}
+
+// any D and group size: one value per thread
+template <int BITS>
+__global__ __launch_bounds__(256) void dequantize_kv_kernel(const uint8_t* __restrict__ codes,
+                                                            const uint16_t* __restrict__ scales,
+                                                            f16* __restrict__ out, int64_t rows, int D, int gs) {
+  const int G = (D + gs - 1) / gs;
+  const int dp = BITS == 8 ? D : (D + 1) / 2;
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < rows * D; i += (int64_t)gridDim.x * 256) {
+    const int64_t r = i / D;
+    const int d = (int)(i - r * D);
+    const uint32_t b = codes[r * dp + (BITS == 8 ? d : d >> 1)];
+    const uint32_t c = BITS == 8 ? b : (d & 1 ? b >> 4 : b & 15u);
+    const float s = fabsf((float)bitcast<f16>(scales[r * G + d / gs]));
+    out[i] = (f16)(((float)c - (BITS == 8 ? 128.0f : 8.0f)) * s);
+  }
+}
+
+// log2 of the 8-value chunks per group when the vector kernels apply (rows of
+// whole groups of 8 .. 512 values, a power of two), else -1
+inline int kv_group_chunks_log2(int64_t D, int64_t gs) {
+  if (gs % 8 || D % gs) return -1;
+  const int64_t l = gs / 8;
+  if (l > MK_WAVE || (l & (l - 1))) return -1;
+  return __builtin_ctzll((unsigned long long)l);
+}
+
+// chunks of 256 threads per launch: far below the grid limit of 2^31 - 1
+constexpr int64_t kMaxKvChunks = (int64_t)256 << 30;
+
 }  // namespace
 
 extern "C" {
@@ -320,6 +427,23 @@ int mk_quantize_kv(const void* src, uint8_t* codes, f16_storage_t* scales, int64
   MK_REQUIRE(D < (1 << 20));
   if (rows == 0) return MK_OK;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const int lgl = kv_group_chunks_log2(D, group_size);
+  if (lgl >= 0 && rows * (D / 8) <= kMaxKvChunks && mk_aligned(src, 16) && mk_aligned(codes, 8)) {
+    const int64_t chunks = rows * (D / 8);
+    const unsigned blocks = (unsigned)((chunks + 255) / 256);
+#define MK_QKV(T, BB) \
+  quantize_kv_vec_kernel<T, BB><<<blocks, 256, 0, st>>>((const T*)src, codes, scales, chunks, lgl)
+    if (dtype == MK_DT_F16) {
+      if (bits == 8) MK_QKV(f16, 8);
+      else MK_QKV(f16, 4);
+    } else {
+      if (bits == 8) MK_QKV(bf16, 8);
+      else MK_QKV(bf16, 4);
+    }
+#undef MK_QKV
+    MK_CHECK_LAUNCH();
+    return MK_OK;
+  }
   const dim3 grid((unsigned)((rows + 255) / 256));
 #define MK_QKV(T, BB)                                                                 \
   quantize_kv_rows_kernel<T, BB><<<grid, 256, 0, st>>>((const T*)src, codes, scales, rows, \
@@ -332,6 +456,30 @@ int mk_quantize_kv(const void* src, uint8_t* codes, f16_storage_t* scales, int64
     else MK_QKV(bf16, 4);
   }
 #undef MK_QKV
+  MK_CHECK_LAUNCH();
+  return MK_OK;
+}
+
+int mk_dequantize_kv(const uint8_t* codes, const f16_storage_t* scales, void* out, int64_t rows, int64_t D,
+                     int64_t group_size, int bits, void* stream) {
+  MK_REQUIRE(codes && scales && out && rows >= 0 && D > 0 && group_size > 0);
+  MK_REQUIRE(bits == 4 || bits == 8);
+  MK_REQUIRE(D < (1 << 20) && group_size < (1LL << 31));
+  if (rows == 0) return MK_OK;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  f16* o = reinterpret_cast<f16*>(out);
+  const int lgl = kv_group_chunks_log2(D, group_size);
+  if (lgl >= 0 && rows * (D / 8) <= kMaxKvChunks && mk_aligned(out, 16) && mk_aligned(codes, 8)) {
+    const int64_t chunks = rows * (D / 8);
+    const unsigned blocks = (unsigned)((chunks + 255) / 256);
+    if (bits == 8) dequantize_kv_vec_kernel<8><<<blocks, 256, 0, st>>>(codes, scales, o, chunks, lgl);
+    else dequantize_kv_vec_kernel<4><<<blocks, 256, 0, st>>>(codes, scales, o, chunks, lgl);
+  } else {
+    const int64_t want = (rows * D + 255) / 256;
+    const unsigned blocks = (unsigned)(want < 65536 ? want : 65536);
+    if (bits == 8) dequantize_kv_kernel<8><<<blocks, 256, 0, st>>>(codes, scales, o, rows, (int)D, (int)group_size);
+    else dequantize_kv_kernel<4><<<blocks, 256, 0, st>>>(codes, scales, o, rows, (int)D, (int)group_size);
+  }
   MK_CHECK_LAUNCH();
   return MK_OK;
 }

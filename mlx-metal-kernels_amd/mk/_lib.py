@@ -70,6 +70,7 @@ SIGNATURES: dict[str, list] = {
     "mk_qkv_rope_paged_update": [_P] * 8 + [_I64] * 8 + [_I, _P],
     "mk_qkv_rope_paged_update_quant": [_P] * 10 + [_I64] * 9 + [_I, _I, _P],
     "mk_quantize_kv": [_P, _P, _P, _I64, _I64, _I64, _I, _I, _P],
+    "mk_dequantize_kv": [_P, _P, _P, _I64, _I64, _I64, _I, _P],
     "mk_paged_attention_workspace_bytes": [_I64] * 6,
     "mk_paged_decode_attention": [_P] * 6 + [_I64] * 7 + [_F, _I, _P, _SZ, _P],
     "mk_paged_decode_attention_noalloc": [_P] * 6 + [_I64] * 7 + [_F, _I, _P],
@@ -112,7 +113,9 @@ def load() -> ctypes.CDLL:
             )
         lib = ctypes.CDLL(str(path), mode=ctypes.RTLD_GLOBAL)
         for name, argtypes in SIGNATURES.items():
-            fn = getattr(lib, name)
+            fn = getattr(lib, name, None)
+            if fn is None:
+                raise NativeLibraryError(f"{path} has no entry point {name}; rebuild the library")
             fn.argtypes = argtypes
             fn.restype = _RESTYPES.get(name, _I)
         found = lib.mk_abi_version()

@@ -234,6 +234,26 @@ def _hip_quantize_rows(pages: torch.Tensor, group_size: int, bits: int):
     return codes, scales
 
 
+def _hip_dequantize(codes: torch.Tensor, scales: torch.Tensor, group_size: int, bits: int, D: int):
+    """mk_dequantize_kv of device codes [..., D | ceil(D/2)] with fp16 scales
+    [..., ceil(D/group_size)] -> fp16 [..., D]; None for what the kernel does
+    not take (host tensors, other types or layouts, scales that need a
+    gradient), which stays with the tensor ops."""
+    want = tuple(codes.shape[:-1])
+    if (codes.device.type != "cuda" or scales.device != codes.device or codes.dtype != torch.uint8
+            or scales.dtype != torch.float16 or (scales.requires_grad and torch.is_grad_enabled()) or D <= 0
+            or group_size <= 0 or tuple(codes.shape) != want + (D if bits == 8 else (D + 1) // 2,)
+            or tuple(scales.shape) != want + ((D + group_size - 1) // group_size,)):
+        return None
+    codes, scales = codes.contiguous(), scales.contiguous()
+    out = torch.empty(want + (D,), dtype=torch.float16, device=codes.device)
+    if out.numel() == 0:
+        return out
+    _lib.launch("mk_dequantize_kv", codes.device, _lib.ptr(codes), _lib.ptr(scales), _lib.ptr(out), out.numel() // D, D,
+                group_size, bits)
+    return out
+
+
 def _unpacked_codes(paged_qkv: PagedQuantizedKVCache, which: str, D: int) -> torch.Tensor:
     codes = paged_qkv.k_pages_q if which == "k" else paged_qkv.v_pages_q
     if paged_qkv.bits == 8:
@@ -249,10 +269,16 @@ def dequantize_kv_pages(paged_qkv: PagedQuantizedKVCache):
     if orig is None:
         raise ValueError("original_page_shape is required for dequantization")
     D = orig[3]
-    K = _dequant_last_dim(_unpacked_codes(paged_qkv, "k", D), paged_qkv.k_scales, paged_qkv.group_size,
-                          paged_qkv.bits, D).to(torch.float16)
-    V = _dequant_last_dim(_unpacked_codes(paged_qkv, "v", D), paged_qkv.v_scales, paged_qkv.group_size,
-                          paged_qkv.bits, D).to(torch.float16)
+
+    def values(which, codes, scales):
+        out = _hip_dequantize(codes, scales, paged_qkv.group_size, paged_qkv.bits, D)
+        if out is None:
+            out = _dequant_last_dim(_unpacked_codes(paged_qkv, which, D), scales, paged_qkv.group_size,
+                                    paged_qkv.bits, D).to(torch.float16)
+        return out
+
+    K = values("k", paged_qkv.k_pages_q, paged_qkv.k_scales)
+    V = values("v", paged_qkv.v_pages_q, paged_qkv.v_scales)
     return K, V
 
 

@@ -30,6 +30,7 @@ from .kv_cache_ops import normalize_positions
 from .paged_kv_ops import _masked_attention
 from .paged_quantized_kv_ops import (
     _dequant_last_dim,
+    _hip_dequantize,
     _hip_quantize_rows,
     _pack_last_dim,
     _quantize_last_dim,
@@ -170,8 +171,13 @@ def dequantize_kv_cache(qkv_cache: QuantizedKVCache):
     qkv_cache = qkv_cache.validate()
     B, S, H, D = _geometry(qkv_cache)
     g, bits = qkv_cache.group_size, qkv_cache.bits
-    K = _dequant_last_dim(_codes(qkv_cache, "k", D), qkv_cache.k_scales, g, bits, D).to(torch.float16)
-    V = _dequant_last_dim(_codes(qkv_cache, "v", D), qkv_cache.v_scales, g, bits, D).to(torch.float16)
+
+    def values(which, codes, scales):
+        out = _hip_dequantize(codes, scales, g, bits, D)
+        return _dequant_last_dim(_codes(qkv_cache, which, D), scales, g, bits, D).to(torch.float16) if out is None else out
+
+    K = values("k", qkv_cache.k_q, qkv_cache.k_scales)
+    V = values("v", qkv_cache.v_q, qkv_cache.v_scales)
     return K, V
 
 
