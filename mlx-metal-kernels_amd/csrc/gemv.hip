@@ -6,9 +6,10 @@
 // q4 codes are packed two per byte (low nibble = even k), so on little-endian
 // hardware a 32-bit word holds 8 consecutive codes, nibble i at bits 4i.
 //
-// Decode batches of at most 4 rows (q8: 2) with fp16 activations and scales
-// take the v_dot2 kernel below, 17-32 rows the two-column-tile kernel;
-// the rest, bf16 and fp32 scales the MFMA path:
+// 33 and more rows take the product kernel (gemm.hip).  Decode batches of at
+// most 4 rows (q8: 2) with fp16 activations and scales take the v_dot2 kernel
+// below, 17-32 rows the two-column-tile kernel; the rest, bf16 and fp32
+// scales the MFMA path:
 // Fast path (M <= 16 per launch, K % 64 == 0 for q4 / % 32 for q8, power-of-two
 // group size >= 16 (q4) / >= 8 (q8)):
 //   * one workgroup owns a 16-row output tile; its KW waves split K;
@@ -26,362 +27,13 @@
 // The MFMA contraction is order-free in k, so the activation operand is built
 // in the same permuted k order the magic unpack produces.
 #include "common.h"
+#include "gemv_common.h"
 #include "norm_chunks.h"
 #include "paged_common.h"
 
+using namespace mkq;
+
 namespace {
-
-constexpr int EPI_NONE = 0;
-constexpr int EPI_RESIDUAL = 1;
-constexpr int EPI_GATE_UP = 2;
-constexpr int EPI_ROPE_KV = 3;  // qkv rows -> split + interleaved RoPE + paged K/V write
-
-template <int BITS>
-struct QFmt {
-  static constexpr int KL = BITS == 4 ? 64 : 32;     // k per lane chunk (32 code bytes)
-  static constexpr int KC = 4 * KL;                  // k per wave chunk
-  static constexpr int STEPS = BITS == 4 ? 8 : 4;    // MFMA k32 steps per chunk
-  static constexpr int ROW_BYTES_NUM = BITS;         // row bytes = K * BITS / 8
-};
-
-// --------------------------------------------------------------------------
-// activation operand: 8 halves of x for one MFMA step, in the k order the
-// weight unpack produces.
-// --------------------------------------------------------------------------
-template <int BITS, bool MAGIC>
-__device__ __forceinline__ u32x4 xperm(u32x4 X) {
-  if constexpr (!MAGIC) {
-    return X;  // natural order
-  } else if constexpr (BITS == 4) {
-    // weight order [0,4,1,5,2,6,3,7]
-    u32x4 r;
-    r[0] = pack_lo16(X[0], X[2]);
-    r[1] = pack_hi16(X[0], X[2]);
-    r[2] = pack_lo16(X[1], X[3]);
-    r[3] = pack_hi16(X[1], X[3]);
-    return r;
-  } else {
-    // weight order [0,2,1,3,4,6,5,7]
-    u32x4 r;
-    r[0] = pack_lo16(X[0], X[1]);
-    r[1] = pack_hi16(X[0], X[1]);
-    r[2] = pack_lo16(X[2], X[3]);
-    r[3] = pack_hi16(X[2], X[3]);
-    return r;
-  }
-}
-
-// Per-group dequant parameters.  The integer part zi of the zero point is
-// subtracted exactly from the magic-biased codes: (1024 + c) - (1024 + zi)
-// for codes at mantissa bits 0..3 (q8: 0..7) of 1024.0h, (64 + c) - (64 + zi)
-// for q4 codes left in place at bits 4..7 under 64.0h (ulp 1/16) -- c - zi
-// exactly in fp16 for |zi| < 1024 -- so w = fma(c - zi, s, corr) with
-// corr = -(z - zi) s rounds once, to the fp16 of (c - z) s whenever z is an
-// integer (the rounding of the reference's fp32 dequant, for any fp16 scale),
-// and keeps a fractional z exact to ulp(corr).
-struct GpMagic {
-  f16x2 s;     // (s, s)
-  f16x2 kz;    // (1024 + zi)
-  f16x2 kz64;  // (64 + zi)
-  f16x2 corr;  // -(z - zi) * s
-};
-struct GpExact {
-  float s;
-  float z;
-};
-
-__device__ __forceinline__ f16x2 h2(f16 v) { return (f16x2){v, v}; }
-
-__device__ __forceinline__ GpMagic make_gp_magic(f16 s, f16 z) {
-  GpMagic g;
-  const float zf = (float)z;
-  const float zi = rintf(zf);
-  g.s = h2(s);
-  g.kz = h2((f16)(1024.0f + zi));
-  g.kz64 = h2((f16)(64.0f + zi));
-  g.corr = h2((f16)(-(zf - zi) * (float)s));
-  return g;
-}
-
-// q4 word (8 codes) -> 8 fp16 weights in order [0,4,1,5,2,6,3,7].
-// `magic` = 0x64006400 (1024.0h pair) and `magic_hi` = 0x54005400 (64.0h
-// pair) held in VGPRs so each unpack is one v_and_or_b32.
-__device__ __forceinline__ u32x4 dq4_magic(uint32_t u, const GpMagic& g, uint32_t magic, uint32_t magic_hi) {
-  const uint32_t v = u >> 8;
-  f16x2 a = bitcast<f16x2>((u & 0x000F000Fu) | magic) - g.kz;       // c0 - zi, c4 - zi
-  f16x2 b = bitcast<f16x2>((u & 0x00F000F0u) | magic_hi) - g.kz64;  // c1 - zi, c5 - zi
-  f16x2 c = bitcast<f16x2>((v & 0x000F000Fu) | magic) - g.kz;       // c2, c6
-  f16x2 d = bitcast<f16x2>((v & 0x00F000F0u) | magic_hi) - g.kz64;  // c3, c7
-  a = __builtin_elementwise_fma(a, g.s, g.corr);
-  b = __builtin_elementwise_fma(b, g.s, g.corr);
-  c = __builtin_elementwise_fma(c, g.s, g.corr);
-  d = __builtin_elementwise_fma(d, g.s, g.corr);
-  u32x4 r;
-  r[0] = bitcast<uint32_t>(a);
-  r[1] = bitcast<uint32_t>(b);
-  r[2] = bitcast<uint32_t>(c);
-  r[3] = bitcast<uint32_t>(d);
-  return r;
-}
-
-// byte-pair unpack of q8 codes with v_perm_b32: bytes (b0, 0x64, b2, 0x64)
-// and (b1, 0x64, b3, 0x64) of {magic8 = 0x64646464, u} are 1024+b0 / 1024+b2
-// and 1024+b1 / 1024+b3 as fp16 pairs.
-__device__ __forceinline__ uint32_t q8_lo_pair(uint32_t u, uint32_t magic8) {
-  return perm_b32(magic8, u, 0x04020400u);
-}
-__device__ __forceinline__ uint32_t q8_hi_pair(uint32_t u, uint32_t magic8) {
-  return perm_b32(magic8, u, 0x04030401u);
-}
-
-// two q8 words (8 codes) -> 8 fp16 weights in order [0,2,1,3,4,6,5,7].
-__device__ __forceinline__ u32x4 dq8_magic(uint32_t u0, uint32_t u1, const GpMagic& g,
-                                           uint32_t magic8) {
-  f16x2 a0 = bitcast<f16x2>(q8_lo_pair(u0, magic8)) - g.kz;
-  f16x2 b0 = bitcast<f16x2>(q8_hi_pair(u0, magic8)) - g.kz;
-  f16x2 a1 = bitcast<f16x2>(q8_lo_pair(u1, magic8)) - g.kz;
-  f16x2 b1 = bitcast<f16x2>(q8_hi_pair(u1, magic8)) - g.kz;
-  a0 = __builtin_elementwise_fma(a0, g.s, g.corr);
-  b0 = __builtin_elementwise_fma(b0, g.s, g.corr);
-  a1 = __builtin_elementwise_fma(a1, g.s, g.corr);
-  b1 = __builtin_elementwise_fma(b1, g.s, g.corr);
-  u32x4 r;
-  r[0] = bitcast<uint32_t>(a0);
-  r[1] = bitcast<uint32_t>(b0);
-  r[2] = bitcast<uint32_t>(a1);
-  r[3] = bitcast<uint32_t>(b1);
-  return r;
-}
-
-// Exact path: w = AT((q - z) * s) computed in fp32, natural k order.
-template <typename AT>
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  AT a = from_f32<AT>(lo), b = from_f32<AT>(hi);
-  return (uint32_t)bitcast<uint16_t>(a) | ((uint32_t)bitcast<uint16_t>(b) << 16);
-}
-
-template <typename AT>
-__device__ __forceinline__ u32x4 dq4_exact(uint32_t u, const GpExact& g) {
-  float w[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) w[e] = ((float)((u >> (4 * e)) & 15u) - g.z) * g.s;
-  u32x4 r;
-#pragma unroll
-  for (int p = 0; p < 4; ++p) r[p] = pack2<AT>(w[2 * p], w[2 * p + 1]);
-  return r;
-}
-
-template <typename AT>
-__device__ __forceinline__ u32x4 dq8_exact(uint32_t u0, uint32_t u1, const GpExact& g) {
-  float w[8];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) w[e] = ((float)((u0 >> (8 * e)) & 255u) - g.z) * g.s;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) w[4 + e] = ((float)((u1 >> (8 * e)) & 255u) - g.z) * g.s;
-  u32x4 r;
-#pragma unroll
-  for (int p = 0; p < 4; ++p) r[p] = pack2<AT>(w[2 * p], w[2 * p + 1]);
-  return r;
-}
-
-template <typename AT>
-__device__ __forceinline__ f32x4 mfma_k32(u32x4 a, u32x4 b, f32x4 c);
-
-template <>
-__device__ __forceinline__ f32x4 mfma_k32<f16>(u32x4 a, u32x4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(bitcast<f16x8>(a), bitcast<f16x8>(b), c, 0, 0, 0);
-}
-template <>
-__device__ __forceinline__ f32x4 mfma_k32<bf16>(u32x4 a, u32x4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8>(a), bitcast<bf16x8>(b), c, 0, 0,
-                                                 0);
-}
-
-template <typename ST>
-__device__ __forceinline__ float ld_scalar_f32(const ST* p) {
-  return to_f32(*p);
-}
-
-// The decode token's cache write fused into the qkv projection's epilogue
-// (EPI_ROPE_KV): the operands of qkv_rope_update_kernel.
-struct RopeKV {
-  const float* cos_t;   // [cos_rows, D/2]
-  const float* sin_t;
-  const int32_t* pos;   // [M]
-  const int32_t* bt;    // [M, max_blocks]
-  void* kp;             // [num_pages, P, Hkv, D] f16
-  void* vp;
-  void* q_out;          // [M, Hq, D] f16
-  int Hq, Hkv, D, P, max_blocks, num_pages, cos_rows;
-};
-
-struct GemvArgs {
-  const void* x;         // [M, K]
-  const uint8_t* w[2];   // [N, row_bytes]
-  const void* s[2];      // [N, G]
-  const void* z[2];      // [N, G] or null
-  const void* residual;  // [M, N] or null
-  void* y0;              // EPI_NONE: y; EPI_RESIDUAL: y_mm (nullable); GATE_UP: gate (nullable)
-  void* y1;              // EPI_RESIDUAL: out;  GATE_UP: up (nullable)
-  void* y2;              // GATE_UP: mlp (nullable)
-  int M, N, K;
-  int row_bytes;
-  int G;
-  int lg;                // log2(group size)
-  int kw;                // waves per row group (K split)
-  int rg;                // dot kernel: row groups per workgroup
-  // residual + RMSNorm prologue (NORM dot kernels, M = 1): the product is
-  // taken against n = fp16(z * rsqrt(mean(z^2) + eps) * nw), z = fp16(x +
-  // nres) (z = x when nres is null); workgroup 0 writes z and n when zout /
-  // nout are given
-  const void* nres;      // [K] or null
-  const void* nw;        // [K] fp16
-  void* zout;            // [K]
-  void* nout;            // [K] or null
-  float eps;
-  RopeKV rk;             // EPI_ROPE_KV only
-};
-
-// --------------------------------------------------------------------------
-// shared epilogue: value(s) of output row n for activation row m
-// --------------------------------------------------------------------------
-template <typename AT, int EPI>
-__device__ __forceinline__ void store_out(const GemvArgs& args, size_t o, float v0, float v1) {
-  if constexpr (EPI == EPI_NONE) {
-    reinterpret_cast<AT*>(args.y0)[o] = saturate_cast<AT>(v0);
-  } else if constexpr (EPI == EPI_RESIDUAL) {
-    const AT d = saturate_cast<AT>(v0);
-    if (args.y0) reinterpret_cast<AT*>(args.y0)[o] = d;
-    const float r = to_f32(reinterpret_cast<const AT*>(args.residual)[o]);
-    reinterpret_cast<AT*>(args.y1)[o] = from_f32<AT>(r + to_f32(d));
-  } else {
-    const AT g = saturate_cast<AT>(v0);
-    const AT u = saturate_cast<AT>(v1);
-    if (args.y0) reinterpret_cast<AT*>(args.y0)[o] = g;
-    if (args.y1) reinterpret_cast<AT*>(args.y1)[o] = u;
-    if (args.y2) {
-      const float gf = to_f32(g);
-      const float sil = gf / (1.0f + expf(-gf));
-      reinterpret_cast<AT*>(args.y2)[o] = from_f32<AT>(sil * to_f32(u));
-    }
-  }
-}
-
-// EPI_ROPE_KV: the launch's rows' cache slots (page * P + offset, -1 when
-// skipped), looked up once per workgroup before its reduction barrier, so the
-// later-row-wins rule reads LDS in the epilogue (rows <= 32 per launch).
-constexpr int kRopeRows = 32;
-__device__ __forceinline__ void rope_fill_slots(const GemvArgs& a, int* slots) {
-  const int t = threadIdx.x;
-  if (t < a.M && t < kRopeRows) {
-    const RopeKV& r = a.rk;
-    int off;
-    const int pg = slot_page(r.bt, r.pos, t, r.max_blocks, r.P, r.num_pages, &off);
-    slots[t] = pg < 0 ? -1 : pg * r.P + off;
-  }
-}
-// this row's slot, or -1 when skipped or taken by a later row of the launch
-__device__ __forceinline__ int rope_slot(const GemvArgs& a, const int* slots, int m) {
-  const int sl = slots[m];
-  if (sl < 0) return -1;
-  for (int b2 = m + 1; b2 < a.M; ++b2)
-    if (slots[b2] == sl) return -1;
-  return sl;
-}
-
-// EPI_ROPE_KV: qkv output n of row m, rounded as the projection stores it,
-// then the arithmetic of qkv_rope_update_kernel -- q and k pairs (n, n ^ 1)
-// rotated in fp32 and rounded, v copied; q to q_out, k and v to the token's
-// cache slot unless its position is out of range or a later row takes the
-// slot.  Called by every lane of the pair (the partner value comes by
-// shuffle), whether or not (m, n) is in range.
-__device__ __forceinline__ void rope_kv_store(const GemvArgs& a, const int* slots, int m, int n, float v) {
-  const f16 hv = saturate_cast<f16>(v);
-  const float xv = to_f32(hv);
-  const float xo = __shfl_xor(xv, 1, 64);
-  if (n >= a.N || m >= a.M) return;
-  const RopeKV& r = a.rk;
-  const int p = r.pos[m];
-  if (p < 0 || p >= r.cos_rows) return;
-  const int D = r.D, QD = r.Hq * D, KD = r.Hkv * D;
-  const int d = n % D;
-  f16 out = hv;
-  f16* dst = reinterpret_cast<f16*>(r.vp);
-  int h;
-  if (n < QD + KD) {
-    const bool even = (d & 1) == 0;
-    const size_t ci = (size_t)p * (D / 2) + (d >> 1);
-    float ye, yo;
-    rope_pair(even ? xv : xo, even ? xo : xv, r.cos_t[ci], r.sin_t[ci], &ye, &yo);
-    out = from_f32<f16>(even ? ye : yo);
-    if (n < QD) {
-      reinterpret_cast<f16*>(r.q_out)[(size_t)m * QD + n] = out;
-      return;
-    }
-    dst = reinterpret_cast<f16*>(r.kp);
-    h = (n - QD) / D;
-  } else {
-    h = (n - QD - KD) / D;
-  }
-  const int sl = rope_slot(a, slots, m);
-  if (sl < 0) return;
-  dst[(size_t)sl * KD + (size_t)h * D + d] = out;
-}
-
-// EPI_ROPE_KV with both values of an (even n, n + 1) pair in one lane (the
-// MFMA kernels' output layout): the same arithmetic as rope_kv_store.  RES:
-// slots[m] already holds the row's final slot (-1 when skipped or taken by a
-// later row) and pos_l[m] its position, both in LDS.
-template <bool RES = false>
-__device__ __forceinline__ void rope_kv_pair(const GemvArgs& a, const int* slots, int m, int n, float v0,
-                                             float v1, const int* pos_l = nullptr) {
-  if (n >= a.N || m >= a.M) return;
-  const RopeKV& r = a.rk;
-  const int p = RES ? pos_l[m] : r.pos[m];
-  if (p < 0 || p >= r.cos_rows) return;
-  const int D = r.D, QD = r.Hq * D, KD = r.Hkv * D;
-  const int d = n % D;
-  const f16 h0 = saturate_cast<f16>(v0), h1 = saturate_cast<f16>(v1);
-  f16 o0 = h0, o1 = h1;
-  f16* dst = reinterpret_cast<f16*>(r.vp);
-  int h;
-  if (n < QD + KD) {
-    const size_t ci = (size_t)p * (D / 2) + (d >> 1);
-    float ye, yo;
-    rope_pair(to_f32(h0), to_f32(h1), r.cos_t[ci], r.sin_t[ci], &ye, &yo);
-    o0 = from_f32<f16>(ye);
-    o1 = from_f32<f16>(yo);
-    if (n < QD) {
-      f16* q = reinterpret_cast<f16*>(r.q_out) + (size_t)m * QD + n;
-      q[0] = o0;
-      q[1] = o1;
-      return;
-    }
-    dst = reinterpret_cast<f16*>(r.kp);
-    h = (n - QD) / D;
-  } else {
-    h = (n - QD - KD) / D;
-  }
-  const int sl = RES ? slots[m] : rope_slot(a, slots, m);
-  if (sl < 0) return;
-  f16* o = dst + (size_t)sl * KD + (size_t)h * D + d;
-  o[0] = o0;
-  o[1] = o1;
-}
-
-// The rows' final slots (the later-row-wins rule applied) and positions into
-// LDS: call after rope_fill_slots(a, raw) and a barrier; the values are
-// visible after the next barrier.
-__device__ __forceinline__ void rope_resolve_slots(const GemvArgs& a, const int* raw, int* res, int* pos_l) {
-  const int t = threadIdx.x;
-  if (t < a.M && t < kRopeRows) {
-    int sl = raw[t];
-    for (int b2 = t + 1; b2 < a.M; ++b2)
-      if (raw[b2] == sl) sl = -1;
-    res[t] = sl;
-    pos_l[t] = a.rk.pos[t];
-  }
-}
 
 // --------------------------------------------------------------------------
 // fast MFMA kernel (any M <= 16)
@@ -1659,19 +1311,6 @@ int launch_tile(GemvArgs a, hipStream_t st) {
   return MK_OK;
 }
 
-// CUs of the current device, cached per device.
-inline int gemv_device_cus() {
-  static int cache[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cache[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cache[dev] = n;
-  }
-  return cache[dev];
-}
-
 // the activation-stationary kernel takes 5..32-row batches of matrices with at
 // least this many 16-row tiles, one per CU (measured against the K-split
 // kernel at 8 / 16 / 32 rows, us: 4096 x 4096 7.05 / 8.2 / 12.8 against 7.5 /
@@ -1715,7 +1354,7 @@ inline size_t xs_lds_bytes(int nw, int nmat, int mt, int G) {
 template <int NMAT, int MT, int EPI>
 int launch_xs(GemvArgs a, hipStream_t st) {
   const int tiles = (a.N + 15) / 16;
-  const int cus = gemv_device_cus();
+  const int cus = device_cu_count();
   const int tpw = (tiles + cus - 1) / cus;
   a.rg = tpw;
   a.kw = a.K / 256;
@@ -1856,6 +1495,10 @@ inline int dot_waves(int64_t K) {
   return (int)(kwd < 1 ? 1 : (kwd > 8 ? 8 : kwd));
 }
 
+// rows from which the matrix-product kernel takes a launch (below: passes of
+// up to 32 rows through the kernels here)
+constexpr int64_t kGemmMinRows = 33;
+
 template <int BITS, int NMAT, int EPI>
 int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int act_dt, int sc_dt,
                   hipStream_t st) {
@@ -1891,6 +1534,20 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
   if constexpr (EPI == EPI_ROPE_KV) {
     // fp16 projections on the fast layouts only (the caller falls back)
     if (act_dt != MK_DT_F16 || sc_dt != MK_DT_F16 || !fast) return MK_ERR_UNSUPPORTED;
+  }
+  if constexpr (EPI != EPI_ROPE_KV) {
+    // One product of all rows, unless two passes of the q4 single-matrix
+    // kernels below take less: few output rows over a long K leave the
+    // product 64 workgroups (4096 x 14336 at 40 rows 66 us against 53; a
+    // pass of 17-32 rows measured 34 us there and 13 at 4096 x 4096).
+    bool product = M >= kGemmMinRows && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
+    if (product && M <= 64 && xk_eligible<BITS, NMAT>(a, 2, act_dt, sc_dt))
+      product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 2.0f * (5.0f + 4.9e-7f * (float)N * (float)K);
+    if (product) {
+      GemvArgs b = a;
+      b.M = (int)M;
+      return launch_gemm_rows<BITS, NMAT, NMAT == 1 ? EPI_RESIDUAL : EPI>(b, act_dt, sc_dt, st);
+    }
   }
   int64_t m_done = 0;
   // up to 32 rows at a time through the activation-stationary kernel
@@ -2168,7 +1825,10 @@ int norm_qkv_rope_entry(const void* x, const void* norm_w, float eps, const uint
     GemvArgs probe = a;
     bool fast;
     gemv_prepare<BITS, 1>(probe, N, K, gs, &fast);
-    if (fast) {
+    // from kGemmMinRows rows on, one product of all rows and the update kernel
+    // beat passes of 32 rows with the update in their epilogue (same bytes)
+    const bool product = M >= kGemmMinRows && gemm_rows_ok<BITS, 1>(probe, M, gs);
+    if (fast && !product) {
       int rc = mk_rms_norm(x, norm_w, normed_out, M, K, eps, act_dt, nw_dt, stream);
       if (rc != MK_OK) return rc;
       return gemv_dispatch<BITS, 1, EPI_ROPE_KV>(a, M, N, K, gs, act_dt, sc_dt, reinterpret_cast<hipStream_t>(stream));

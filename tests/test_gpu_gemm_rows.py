@@ -1,0 +1,107 @@
+"""The matrix-product kernel (33 and more activation rows): every workgroup
+shape, tile edges in rows, output rows and K, types, group sizes and scale
+layouts, against a float64 product of the weights as the reference rounds
+them (to the activation type, ops/quant_ops.py:509-526).
+
+Bound: fp32 accumulation of K products, each partial sum within 2^-24 of it
+(K * 2^-24 * sum |x||w| over any order), then one rounding to the type."""
+
+import pytest
+import torch
+
+import mk.quant_ops as qo
+
+pytestmark = pytest.mark.gpu
+
+HALF_ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _weight(gen, dev, N, K, bits, g, sdt, zeros):
+    top = 16 if bits == 4 else 256
+    codes = torch.randint(0, top, (N, K), generator=gen, device=dev, dtype=torch.uint8)
+    G = -(-K // g)
+    # fp16 scales and zero points in eighths: (q - z) * s is then exact in
+    # fp32 (22 bits), and the rounded weight does not depend on whether that
+    # product is rounded first
+    s = (torch.rand((N, G), generator=gen, device=dev) * 0.01 + 0.001).half().to(sdt)
+    z = None
+    if zeros == "affine":  # fractional zero points
+        z = (torch.randint(0, 8 * top, (N, G), generator=gen, device=dev) / 8).to(sdt)
+    elif zeros == "whole":
+        z = torch.randint(0, top, (N, G), generator=gen, device=dev).to(sdt)
+    packed = codes
+    if bits == 4:
+        packed = codes[:, 0::2] | (codes[:, 1::2] << 4)
+    return codes, packed.contiguous(), s, z
+
+
+def _rounded(codes, s, z, g, dtype):
+    K = codes.shape[1]
+    full = s.float().repeat_interleave(g, 1)[:, :K]
+    zero = 0.0 if z is None else z.float().repeat_interleave(g, 1)[:, :K]
+    return ((codes.float() - zero) * full).to(dtype).double()
+
+
+def _check(got, x, W, dtype, what):
+    ref = x.double() @ W.t()
+    bound = x.shape[1] * 2.0 ** -24 * (x.double().abs() @ W.abs().t())
+    lim = bound + 1.01 * HALF_ULP[dtype] * ref.abs() + 2.0 ** -24
+    err = (got.double() - ref).abs()
+    assert bool((err <= lim).all()), (what, float((err - lim).max()), float(err.max()))
+
+
+CASES = [  # M, N, K: the smallest; ragged N and K, one past a column tile; tiles of 64 and 128 rows and one more
+    (33, 4, 32), (40, 101, 96), (64, 257, 2080), (65, 515, 1024), (128, 64, 4096), (129, 1030, 512),
+    # many tiles of output rows (8 x 8), few of them over a long K (8 x 1 x 4, 4 x 2 x 4, 4 x 1 x 4), and between (8 x 2 x 2)
+    (509, 14336, 256), (500, 4096, 1056), (256, 2048, 14336), (72, 1024, 7168), (130, 6144, 4096)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K", CASES)
+def test_product_rows(dev, M, N, K, bits, dtype):
+    gen = torch.Generator(device=dev).manual_seed(M * 7 + N + K)
+    x = torch.randn((M, K), generator=gen, device=dev).to(dtype)
+    fn = qo.q4_matvec_decode if bits == 4 else qo.q8_matvec_decode
+    for g, sdt, zeros in ((64, torch.float16, "whole"), (32, torch.float16, "none"), (128, torch.float32, "affine")):
+        codes, packed, s, z = _weight(gen, dev, N, K, bits, g, sdt, zeros)
+        W = _rounded(codes, s, z, g, dtype)
+        got = fn(x, packed, s, z, group_size=g)
+        _check(got, x, W, dtype, f"M{M} N{N} K{K} q{bits} g{g} {sdt} {zeros}")
+        res = torch.randn((M, N), generator=gen, device=dev).to(dtype)
+        mm, out = qo.q_matvec_residual(x, packed, s, z, res, bits=bits, group_size=g, want_mm=True)
+        assert torch.equal(mm, got)
+        assert torch.equal(out, (res.float() + mm.float()).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K", [(33, 7, 64), (65, 260, 160), (200, 1024, 1024), (509, 14336, 128)])
+def test_product_gate_up(dev, M, N, K, bits, dtype):
+    gen = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen, device=dev).to(dtype)
+    cg, gw, gs, gz = _weight(gen, dev, N, K, bits, 32, torch.float16, "whole")
+    cu, uw, us, uz = _weight(gen, dev, N, K, bits, 32, torch.float16, "whole")
+    gate, up, mlp = qo.q_gate_up_swiglu(x, gw, uw, gs, us, gz, uz, bits=bits, group_size=32, return_gate_up=True)
+    _check(gate, x, _rounded(cg, gs, gz, 32, dtype), dtype, "gate")
+    _check(up, x, _rounded(cu, us, uz, 32, dtype), dtype, "up")
+    gf = gate.double()
+    want = gf / (1 + torch.exp(-gf)) * up.double()
+    # silu in fp32 (a few 2^-24), the product rounded once
+    assert bool(((mlp.double() - want).abs() <= 1.01 * HALF_ULP[dtype] * want.abs() + 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_product_unaligned_scales_and_saturation(dev, bits):
+    """Scales 2 bytes off (copied one by one) give the aligned result; sums
+    past fp16 saturate."""
+    gen = torch.Generator(device=dev).manual_seed(3)
+    M, N, K, g = 70, 130, 1024, 64
+    x = torch.randn((M, K), generator=gen, device=dev).half()
+    _, packed, s, z = _weight(gen, dev, N, K, bits, g, torch.float16, "whole")
+    fn = qo.q4_matvec_decode if bits == 4 else qo.q8_matvec_decode
+    want = fn(x, packed, s, z, group_size=g)
+    off = lambda t: torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)[1:].reshape(t.shape).copy_(t)
+    assert torch.equal(fn(x, packed, off(s), off(z), group_size=g), want)
+    big = fn(torch.full((40, K), 200.0, device=dev).half(), packed, s * 400, None, group_size=g)
+    assert bool((big == 65504.0).all())
