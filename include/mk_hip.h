@@ -97,6 +97,19 @@ int mk_q8_matvec(const void* x, const uint8_t* w, const void* scales, const void
                  const void* residual, void* y_mm, void* y_out, int64_t M, int64_t N, int64_t K,
                  int64_t group_size, int act_dtype, int scale_dtype, void* stream);
 
+/* The same with a workspace (16-byte aligned, any content) of
+ * mk_matvec_workspace_bytes(M, N, K) bytes: 0 unless M <= 64 and K > 4096,
+ * where it lets passes of up to 32 rows split K over workgroups (the fp32 sums of the
+ * slices go through it).  Without one such calls take the kernels that walk
+ * whole rows. */
+size_t mk_matvec_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int mk_q4_matvec_ws(const void* x, const uint8_t* w, const void* scales, const void* zeros, const void* residual,
+                    void* y_mm, void* y_out, int64_t M, int64_t N, int64_t K, int64_t group_size, int act_dtype,
+                    int scale_dtype, void* workspace, size_t workspace_bytes, void* stream);
+int mk_q8_matvec_ws(const void* x, const uint8_t* w, const void* scales, const void* zeros, const void* residual,
+                    void* y_mm, void* y_out, int64_t M, int64_t N, int64_t K, int64_t group_size, int act_dtype,
+                    int scale_dtype, void* workspace, size_t workspace_bytes, void* stream);
+
 /* q4_gate_up_matvec_tiled -- ops/quant_ops.py:634-685 (one x read, two weight
  * streams).  gate_out/up_out [M,N] (nullable) receive the two products;
  * mlp_out [M,N] (nullable) receives the fused SwiGLU epilogue

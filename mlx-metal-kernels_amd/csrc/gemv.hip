@@ -368,217 +368,10 @@ __global__ __launch_bounds__(NMAT == 1 && BITS == 4 ? 1024 : 512) void gemv_tile
 }
 
 // --------------------------------------------------------------------------
-// Activation-stationary batched kernel (q4, fp16 activations and scales,
-// 5..32 rows, K % 256 == 0, K <= 4096): the MFMA kernels above re-read each
-// activation row from L2 for every 16-row weight tile, so at 32 rows the
-// activation reads (M x K x 2 bytes per tile) outweigh the 16 x K / 2 code
-// bytes they multiply.  Here a workgroup of K / 256 waves keeps the whole
-// activation block in registers -- wave w holds k in [256 w, 256 w + 256) of
-// every row, lane (r = l % 16, kb = l / 16) two 32-k runs, pre-permuted to
-// the order the weight unpack produces (64 VGPRs at 32 rows) -- and walks a
-// contiguous run of 16-row tiles: per tile each lane loads the 2 x 16 code
-// bytes of row r over its runs, the dequantized operand feeds the MT
-// column tiles' v_mfma_f32_16x16x32_f16 steps, and the K / 256 partial tiles
-// are summed through LDS (double buffered) by MT waves that take turns.  The
-// tile's scales and zero points (16 rows x G, contiguous) are staged in LDS
-// by the whole workgroup, one 16-byte vector per thread, instead of one
-// 2-byte gather per lane and group from every wave (which cost 30.5 against
-// 23.9 us with the gathers replaced by constants, gate/up at 8 rows).  One
-// barrier per tile publishes both the tile's partials and the next tile's
-// (s, z).  Measured, 2 x 14336 x 4096 gate/up + SwiGLU: 19.4 / 21.3 / 27.4 us
-// at 8 / 16 / 32 rows against 31.0 / 36.1 / 57.4 for the kernels above.
-// --------------------------------------------------------------------------
-template <int NMAT>
-struct XsBuf {
-  u32x4 w[NMAT][2];  // 32 code bytes: 64 k of row r
-  u32x4 sz;          // this thread's 16-byte vector of the tile's (s, z) block
-};
-
-// The runs: RUN = 128 puts them at 32 kb and 128 + 32 kb, so each load
-// instruction reads the 16 rows' aligned 64-byte half lines whole (used for
-// one column tile, where it measured 2 % faster); RUN = 32 makes them one
-// 64-k span at 64 kb, whose simpler addressing keeps the two-column-tile
-// kernel within 128 VGPRs.
-template <int NMAT, int MT, int EPI, int RUN>
-__global__ __launch_bounds__(1024) void gemv_xs_kernel(const GemvArgs args) {
-  constexpr int STEPS = 8;  // k32 MFMA steps per lane's 64 k (4 per run)
-  using Buf = XsBuf<NMAT>;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nw = args.kw;  // waves = K / 256
-  const int M = args.M, N = args.N, K = args.K, G = args.G;
-  const int r = lane & 15, kb = lane >> 4;
-  const int tiles = (N + 15) >> 4;
-  const int t_begin = blockIdx.x * args.rg;  // rg: tiles per workgroup
-  const int t_end = min(t_begin + args.rg, tiles);
-  const int ka = wave * 256 + kb * (RUN == 128 ? 32 : 64);  // run a: steps 0-3; run b = ka + RUN: 4-7
-  const uint32_t magic = in_vgpr(0x64006400u);
-  const uint32_t magic_hi = in_vgpr(0x54005400u);  // odd nibbles under 64.0h
-  const bool has_z = args.z[0] != nullptr;
-  const int ga = ka >> args.lg, gb = (ka + RUN) >> args.lg;  // g >= 32: one group per run
-
-  // LDS: [2][nw][NMAT * MT][64] f32x4 partial tiles, then [2][2 NMAT][16][G + 2]
-  // fp16 (s, z) slots (rows padded by 4 bytes: the 16 rows a read touches
-  // fall in 16 banks)
-  extern __shared__ __align__(16) uint8_t xs_lds[];
-  f32x4* red = reinterpret_cast<f32x4*>(xs_lds);
-  const int slab = nw * NMAT * MT * 64;  // f32x4 per partial buffer
-  const int gp = G + 2;
-  f16* szs = reinterpret_cast<f16*>(xs_lds + (size_t)2 * slab * sizeof(f32x4));
-  const int slot_len = 2 * NMAT * 16 * gp;
-
-  // this thread's (s, z) vector: piece p (s0, z0, s1, z1), row, 8 groups at c8
-  const int vec_per_piece = 2 * G;  // 16 rows x G / 8
-  const int nvec = 2 * NMAT * vec_per_piece;
-  const bool sz_live = tid < nvec;
-  const int vt = sz_live ? tid : 0;
-  const int sp = vt / vec_per_piece;
-  const int se = vt - sp * vec_per_piece;
-  const int srow = se / (G >> 3);
-  const int sc8 = se - srow * (G >> 3);
-  const bool s_zero = (sp & 1) && !has_z;  // zero points absent: z = 0
-  const f16* sbase = reinterpret_cast<const f16*>((sp & 1) && has_z ? args.z[sp >> 1] : args.s[sp >> 1]) +
-                     (size_t)srow * G + 8 * sc8;
-  const uint32_t code_off = (uint32_t)r * (uint32_t)args.row_bytes + (uint32_t)(ka >> 1);
-  // EPI_ROPE_KV: the rows' cache slots as looked up, then with the
-  // later-row-wins rule applied, and the rows' positions
-  __shared__ int rk_slots[EPI == EPI_ROPE_KV ? kRopeRows : 1];
-  __shared__ int rk_res[EPI == EPI_ROPE_KV ? kRopeRows : 1];
-  __shared__ int rk_pos[EPI == EPI_ROPE_KV ? kRopeRows : 1];
-
-  // the activation block: column 16 mt + r (rows past M repeat row M - 1;
-  // their results are dropped)
-  u32x4 xp[MT][STEPS];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int m = min(16 * mt + r, M - 1);
-    const f16* xr = reinterpret_cast<const f16*>(args.x) + (size_t)m * K + ka;
-#pragma unroll
-    for (int st = 0; st < STEPS; ++st) xp[mt][st] = xperm<4, true>(ldg128(xr + (st >> 2) * RUN + 8 * (st & 3)));
-  }
-  __builtin_amdgcn_sched_barrier(0);
-
-  // tile t's codes for row r and this thread's (s, z) vector (N % 16 == 0:
-  // every row of a tile exists); tiles past the run re-read its first
-  auto tile_of = [&](int t) { return __builtin_amdgcn_readfirstlane(t < t_end ? t : t_begin); };
-  auto issue_codes = [&](int t, int q, Buf& b) {
-    const uint8_t* p = args.w[q] + (size_t)tile_of(t) * 16 * args.row_bytes + code_off;
-    b.w[q][0] = ldg128_stream(p);
-    b.w[q][1] = ldg128_stream(p + RUN / 2);
-  };
-  auto issue_sz = [&](int t, u32x4& v) { v = ldg128(sbase + (size_t)tile_of(t) * 16 * G); };
-  auto issue = [&](int t, Buf& b) {
-#pragma unroll
-    for (int q = 0; q < NMAT; ++q) issue_codes(t, q, b);
-    issue_sz(t, b.sz);
-  };
-  auto stage_v = [&](const u32x4& v, int slot) {
-    if (sz_live) {
-      uint32_t* d = reinterpret_cast<uint32_t*>(szs + (size_t)(slot & 1) * slot_len + (sp * 16 + srow) * gp + 8 * sc8);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) d[e] = s_zero ? 0u : v[e];
-    }
-  };
-  auto stage = [&](const Buf& b, int slot) { stage_v(b.sz, slot); };
-
-  // one tile: products against the staged (s, z), partials to LDS; the
-  // barrier and the reduction follow in the loop
-  auto compute_q = [&](const Buf& b, int it, int q) {
-    const f16* sl = szs + (size_t)(it & 1) * slot_len + r * gp;
-    f32x4* rb = red + (it & 1) * slab;
-    {
-      f32x4 acc[MT];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int g = h ? gb : ga;
-        const GpMagic gpm = make_gp_magic(sl[(2 * q) * 16 * gp + g], sl[(2 * q + 1) * 16 * gp + g]);
-#pragma unroll
-        for (int st = 4 * h; st < 4 * h + 4; ++st) {
-          const u32x4 a = dq4_magic(b.w[q][h][st & 3], gpm, magic, magic_hi);
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma_k32<f16>(a, xp[mt][st], acc[mt]);
-        }
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) rb[(wave * NMAT * MT + q * MT + mt) * 64 + lane] = acc[mt];
-    }
-  };
-  // the reducing waves sum the nw partials of tile t and store them (lane
-  // holds D[n = 4 kb + i][m = 16 mt + r])
-  auto reduce = [&](int t, int it) {
-    const f32x4* rb = red + (it & 1) * slab;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      if (wave != (it * MT + mt) % nw) continue;
-      const int m = 16 * mt + r;
-      f32x4 v[NMAT];
-#pragma unroll
-      for (int q = 0; q < NMAT; ++q) {
-        v[q] = rb[(q * MT + mt) * 64 + lane];
-        for (int w = 1; w < nw; ++w) v[q] += rb[(w * NMAT * MT + q * MT + mt) * 64 + lane];
-      }
-      const int nb = t * 16 + 4 * kb;
-      if (m < M && t < t_end) {
-        if constexpr (EPI == EPI_ROPE_KV) {  // NMAT == 1; the pairs are (nb, nb+1), (nb+2, nb+3)
-          rope_kv_pair<true>(args, rk_res, m, nb, v[0][0], v[0][1], rk_pos);
-          rope_kv_pair<true>(args, rk_res, m, nb + 2, v[0][2], v[0][3], rk_pos);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int nn = nb + i;
-            if (nn < N) store_out<f16, EPI>(args, (size_t)m * N + nn, v[0][i], v[NMAT - 1][i]);
-          }
-        }
-      }
-    }
-  };
-
-  // One code buffer: each matrix's codes are refilled with the next tile's as
-  // soon as its products are issued, and the (s, z) vector for tile t + 1 is
-  // issued at the start of tile t -- ahead of t + 1's codes, so staging it at
-  // the end of tile t waits for it alone and the barrier never waits for
-  // codes.  (Measured against a ring of two or three code buffers refilled
-  // after a whole tile, whose (s, z) wait also covered the next tile's codes:
-  // 19.4 against 24.0 us for the 2 x 14336 x 4096 gate/up at 8 rows.)  The
-  // loop refills the same registers in place every iteration, so no buffer
-  // is copied across it.  The steps for a tile past the run compute on
-  // re-read data and store nothing.
-  // EPI_ROPE_KV: the rows' cache slots, in LDS before the first barrier,
-  // resolved after it (the loop's barrier precedes the first epilogue)
-  if constexpr (EPI == EPI_ROPE_KV) rope_fill_slots(args, rk_slots);
-
-  Buf b;
-  issue(t_begin, b);
-  __builtin_amdgcn_sched_barrier(0);
-  stage(b, 0);
-  __syncthreads();
-  if constexpr (EPI == EPI_ROPE_KV) rope_resolve_slots(args, rk_slots, rk_res, rk_pos);
-  int it = 0;
-  for (int t = t_begin; t < t_end; ++t, ++it) {
-    issue_sz(t + 1, b.sz);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int q = 0; q < NMAT; ++q) {
-      compute_q(b, it, q);
-      __builtin_amdgcn_sched_barrier(0);
-      issue_codes(t + 1, q, b);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    stage(b, it + 1);
-    __syncthreads();
-    reduce(t, it);
-  }
-}
-
-// --------------------------------------------------------------------------
 // K-split batched kernel (q4, fp16 activations and scales, 5..32 rows, one
-// matrix, K % 128 == 0 with 2048 <= K <= 16384, N % 16 == 0): for the
-// matrices the activation-stationary kernel does not take -- long rows (the
-// 14336-k down projection) or too few row tiles to share one activation block
-// (o-proj, qkv).  One 16-row tile per workgroup of 16 waves; wave w takes an
+// matrix, K % 128 == 0 with 2048 <= K <= 16384, N % 16 == 0): long rows (the
+// 14336-k down projection) of calls that give no workspace, which the few-row
+// kernel needs to split them over workgroups.  One 16-row tile per workgroup of 16 waves; wave w takes an
 // equal run of the row's 128-k halves (7 at K = 14336) and requests all of its
 // codes up front (one 16-byte load per half: lane (r, kb) reads k in
 // [128 h + 32 kb, +32) of row r, so each instruction reads the 16 rows'
@@ -1311,13 +1104,8 @@ int launch_tile(GemvArgs a, hipStream_t st) {
   return MK_OK;
 }
 
-// the activation-stationary kernel takes 5..32-row batches of matrices with at
-// least this many 16-row tiles, one per CU (measured against the K-split
-// kernel at 8 / 16 / 32 rows, us: 4096 x 4096 7.05 / 8.2 / 12.8 against 7.5 /
-// 8.65 / 13.0; 6144 x 4096 9.1 / 10.3 / 14.9 against 13.0 / 15.3 / 24.4)
-constexpr int kXsMinRows = 5;
-constexpr int kXsMinTiles = 256;
-constexpr size_t kXsMaxLds = 160 * 1024;
+constexpr int kXkMinRows = 5;  // fewer: the v_dot2 and MFMA kernels
+constexpr size_t kXkMaxLds = 160 * 1024;
 
 // K-split launch: one 16-row tile per workgroup of 16 waves
 template <int MT, int EPI>
@@ -1337,47 +1125,9 @@ bool xk_eligible(const GemvArgs& a, int mt, int act_dt, int sc_dt) {
   const int H = a.K / 128;
   bool ok = BITS == 4 && NMAT == 1 && act_dt == MK_DT_F16 && sc_dt == MK_DT_F16 && a.lg >= 5 &&
             (a.K % 128) == 0 && H >= XK_WAVES && H <= XK_WAVES * XK_MAX_HALVES && (a.N % 16) == 0 &&
-            (a.G % 8) == 0 && 4 * a.G <= 2 * 64 * XK_WAVES && xk_lds_bytes(mt, a.G) <= kXsMaxLds &&
+            (a.G % 8) == 0 && 4 * a.G <= 2 * 64 * XK_WAVES && xk_lds_bytes(mt, a.G) <= kXkMaxLds &&
             mk_aligned(a.x, 16) && (size_t)a.row_bytes % 16 == 0 && mk_aligned(a.w[0], 16) &&
             mk_aligned(a.s[0], 16) && (a.z[0] == nullptr || mk_aligned(a.z[0], 16));
-  return ok;
-}
-
-// partial tiles (double buffered) + two (s, z) slots with 4-byte row padding
-inline size_t xs_lds_bytes(int nw, int nmat, int mt, int G) {
-  return (size_t)2 * nw * nmat * mt * 64 * sizeof(f32x4) + (size_t)2 * 2 * nmat * 16 * (G + 2) * 2;
-}
-
-// Activation-stationary launch: K / 256 waves per workgroup, the 16-row tiles
-// dealt out in equal contiguous runs to at most one workgroup per CU (the
-// 128 KB partial buffer and 16 waves of <= 128 VGPRs fill a CU).
-template <int NMAT, int MT, int EPI>
-int launch_xs(GemvArgs a, hipStream_t st) {
-  const int tiles = (a.N + 15) / 16;
-  const int cus = device_cu_count();
-  const int tpw = (tiles + cus - 1) / cus;
-  a.rg = tpw;
-  a.kw = a.K / 256;
-  const dim3 grid((unsigned)((tiles + tpw - 1) / tpw));
-  const dim3 block((unsigned)(64 * a.kw));
-  const size_t lds = xs_lds_bytes(a.kw, NMAT, MT, a.G);
-  gemv_xs_kernel<NMAT, MT, EPI, MT == 1 ? 128 : 32><<<grid, block, lds, st>>>(a);
-  MK_CHECK_LAUNCH();
-  return MK_OK;
-}
-
-// q4 only, fp16 activations and scales, 256 <= K <= 4096 with K % 256 == 0,
-// power-of-two group >= 32 (one group per lane's 32-k run), 16-byte
-// aligned x and codes, and enough rows that every CU gets tiles to stream
-template <int BITS, int NMAT, int EPI>
-bool xs_eligible(const GemvArgs& a, int mt, int act_dt, int sc_dt) {
-  bool ok = BITS == 4 && (EPI != EPI_ROPE_KV || NMAT == 1) && act_dt == MK_DT_F16 && sc_dt == MK_DT_F16 && a.lg >= 5 &&
-            (a.K % 256) == 0 && a.K >= 256 && a.K <= 4096 &&
-            (a.N % 16) == 0 && a.N / 16 >= kXsMinTiles && mk_aligned(a.x, 16) && (size_t)a.row_bytes % 16 == 0 &&
-            (a.G % 8) == 0 && 4 * NMAT * a.G <= 64 * (a.K / 256) &&  // one (s, z) vector per thread
-            xs_lds_bytes(a.K / 256, NMAT, mt, a.G) <= kXsMaxLds;
-  for (int t = 0; t < NMAT; ++t)
-    ok = ok && mk_aligned(a.w[t], 16) && mk_aligned(a.s[t], 16) && (a.z[0] == nullptr || mk_aligned(a.z[t], 16));
   return ok;
 }
 
@@ -1501,7 +1251,7 @@ constexpr int64_t kGemmMinRows = 33;
 
 template <int BITS, int NMAT, int EPI>
 int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int act_dt, int sc_dt,
-                  hipStream_t st) {
+                  hipStream_t st, float* ws = nullptr, size_t ws_bytes = 0) {
   using F = QFmt<BITS>;
   MK_REQUIRE(M >= 0 && N > 0 && K > 0 && gs > 0);
   MK_REQUIRE(act_dt == MK_DT_F16 || act_dt == MK_DT_BF16);
@@ -1535,39 +1285,48 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
     // fp16 projections on the fast layouts only (the caller falls back)
     if (act_dt != MK_DT_F16 || sc_dt != MK_DT_F16 || !fast) return MK_ERR_UNSUPPORTED;
   }
-  if constexpr (EPI != EPI_ROPE_KV) {
-    // One product of all rows, unless two passes of the q4 single-matrix
-    // kernels below take less: few output rows over a long K leave the
-    // product 64 workgroups (4096 x 14336 at 40 rows 66 us against 53; a
-    // pass of 17-32 rows measured 34 us there and 13 at 4096 x 4096).
-    bool product = M >= kGemmMinRows && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
-    if (product && M <= 64 && xk_eligible<BITS, NMAT>(a, 2, act_dt, sc_dt))
-      product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 2.0f * (5.0f + 4.9e-7f * (float)N * (float)K);
-    if (product) {
-      GemvArgs b = a;
-      b.M = (int)M;
-      return launch_gemm_rows<BITS, NMAT, NMAT == 1 ? EPI_RESIDUAL : EPI>(b, act_dt, sc_dt, st);
+  // The few-row kernel takes up to 32 rows a pass (8-bit codes: 16) of what
+  // the v_dot2 kernel does not.  From kGemmMinRows rows one product of all
+  // rows, unless two passes take less: few output rows over a long K leave the
+  // product 64 workgroups (4096 x 14336 at 40 rows 66 us against 44; a pass of
+  // 17-32 rows takes 4.5 us + 0.30 ns per 1000 weights for q4 fp16, 4 + 0.43
+  // for bf16).  17-32 rows over 8-bit codes: the product for gate/up (two
+  // passes 70 us, the tile kernel 65), two passes for bf16 (47 against 65 at
+  // 4096 x 14336), the tile kernel below for fp16.
+  {
+    constexpr int64_t kPass = BITS == 4 ? 32 : 16;
+    const bool few = M <= 2 * kPass && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
+                     (EPI != EPI_ROPE_KV || act_dt == MK_DT_F16) &&
+                     few_ok<BITS, NMAT>(a, M < kPass ? M : kPass, gs, sc_dt, ws_bytes);
+    const bool wide8 = BITS == 8 && M > kPass;
+    if constexpr (EPI != EPI_ROPE_KV) {
+      bool product = (M >= kGemmMinRows || (wide8 && NMAT == 2)) && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
+      if (product && few && M >= kGemmMinRows && BITS == 4 && NMAT == 1) {
+        const float pass = act_dt == MK_DT_F16 ? 4.5f + 3.0e-7f * (float)N * (float)K : 4.0f + 4.3e-7f * (float)N * (float)K;
+        product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 2.0f * pass;
+      }
+      if (product) {
+        GemvArgs b = a;
+        b.M = (int)M;
+        return launch_gemm_rows<BITS, NMAT, NMAT == 1 ? EPI_RESIDUAL : EPI>(b, act_dt, sc_dt, st);
+      }
+    }
+    if (few && !(wide8 && act_dt == MK_DT_F16)) {
+      for (int64_t m0 = 0; m0 < M && rc == MK_OK; m0 += kPass) {
+        GemvArgs b = a;
+        b.M = (int)(M - m0 < kPass ? M - m0 : kPass);
+        rows_from(b, m0);
+        rc = launch_few<BITS, NMAT, EPI == EPI_NONE ? EPI_RESIDUAL : EPI>(b, act_dt, ws, st);
+      }
+      return rc;
     }
   }
   int64_t m_done = 0;
-  // up to 32 rows at a time through the activation-stationary kernel
-  {
-    if (M >= kXsMinRows && xs_eligible<BITS, NMAT, EPI>(a, 1, act_dt, sc_dt)) {
-      while (M - m_done >= kXsMinRows && rc == MK_OK) {
-        GemvArgs b = a;
-        int64_t mrows = (M - m_done) < 32 ? (M - m_done) : 32;
-        if (mrows > 16 && !xs_eligible<BITS, NMAT, EPI>(a, 2, act_dt, sc_dt)) mrows = 16;
-        b.M = (int)mrows;
-        rows_from(b, m_done);
-        rc = mrows > 16 ? launch_xs<NMAT, 2, EPI>(b, st) : launch_xs<NMAT, 1, EPI>(b, st);
-        m_done += mrows;
-      }
-    }
-  }
-  // otherwise up to 32 rows at a time through the K-split kernel
+  // up to 32 rows at a time through the K-split kernel (long rows without a
+  // workspace)
   if constexpr (NMAT == 1) {
-    if (M - m_done >= kXsMinRows && xk_eligible<BITS, NMAT>(a, 1, act_dt, sc_dt)) {
-      while (M - m_done >= kXsMinRows && rc == MK_OK) {
+    if (M - m_done >= kXkMinRows && xk_eligible<BITS, NMAT>(a, 1, act_dt, sc_dt)) {
+      while (M - m_done >= kXkMinRows && rc == MK_OK) {
         GemvArgs b = a;
         int64_t mrows = (M - m_done) < 32 ? (M - m_done) : 32;
         if (mrows > 16 && !xk_eligible<BITS, NMAT>(a, 2, act_dt, sc_dt)) mrows = 16;
@@ -1630,7 +1389,7 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
 template <int BITS>
 int matvec_entry(const void* x, const uint8_t* w, const void* s, const void* z, const void* residual,
                  void* y_mm, void* y_out, int64_t M, int64_t N, int64_t K, int64_t gs, int act_dt,
-                 int sc_dt, void* stream) {
+                 int sc_dt, void* stream, void* ws = nullptr, size_t ws_bytes = 0) {
   GemvArgs a = {};
   a.x = x;
   a.w[0] = a.w[1] = w;
@@ -1642,12 +1401,12 @@ int matvec_entry(const void* x, const uint8_t* w, const void* s, const void* z, 
     MK_REQUIRE(y_out);
     a.y0 = y_mm;
     a.y1 = y_out;
-    return gemv_dispatch<BITS, 1, EPI_RESIDUAL>(a, M, N, K, gs, act_dt, sc_dt, st);
+    return gemv_dispatch<BITS, 1, EPI_RESIDUAL>(a, M, N, K, gs, act_dt, sc_dt, st, (float*)ws, ws_bytes);
   }
   void* y = y_out ? y_out : y_mm;
   MK_REQUIRE(y);
   a.y0 = y;
-  int rc = gemv_dispatch<BITS, 1, EPI_NONE>(a, M, N, K, gs, act_dt, sc_dt, st);
+  int rc = gemv_dispatch<BITS, 1, EPI_NONE>(a, M, N, K, gs, act_dt, sc_dt, st, (float*)ws, ws_bytes);
   if (rc == MK_OK && y_mm && y_out && y_mm != y_out) {
     hipError_t e = hipMemcpyAsync(y_mm, y_out, (size_t)M * N * 2, hipMemcpyDeviceToDevice, st);
     if (e != hipSuccess) return -(int)e - 1000;
@@ -1896,6 +1655,24 @@ int mk_q8_matvec(const void* x, const uint8_t* w, const void* scales, const void
                  int64_t group_size, int act_dtype, int scale_dtype, void* stream) {
   return matvec_entry<8>(x, w, scales, zeros, residual, y_mm, y_out, M, N, K, group_size, act_dtype,
                          scale_dtype, stream);
+}
+
+size_t mk_matvec_workspace_bytes(int64_t M, int64_t N, int64_t K) { return few_workspace_bytes(M, N, K); }
+
+int mk_q4_matvec_ws(const void* x, const uint8_t* w, const void* scales, const void* zeros, const void* residual,
+                    void* y_mm, void* y_out, int64_t M, int64_t N, int64_t K, int64_t group_size, int act_dtype,
+                    int scale_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  MK_REQUIRE(workspace_bytes == 0 || (workspace && mk_aligned(workspace, 16)));
+  return matvec_entry<4>(x, w, scales, zeros, residual, y_mm, y_out, M, N, K, group_size, act_dtype, scale_dtype,
+                         stream, workspace, workspace_bytes);
+}
+
+int mk_q8_matvec_ws(const void* x, const uint8_t* w, const void* scales, const void* zeros, const void* residual,
+                    void* y_mm, void* y_out, int64_t M, int64_t N, int64_t K, int64_t group_size, int act_dtype,
+                    int scale_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  MK_REQUIRE(workspace_bytes == 0 || (workspace && mk_aligned(workspace, 16)));
+  return matvec_entry<8>(x, w, scales, zeros, residual, y_mm, y_out, M, N, K, group_size, act_dtype, scale_dtype,
+                         stream, workspace, workspace_bytes);
 }
 
 int mk_q4_gate_up(const void* x, const uint8_t* w_gate, const uint8_t* w_up, const void* s_gate,

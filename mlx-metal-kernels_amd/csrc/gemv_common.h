@@ -360,6 +360,87 @@ __device__ __forceinline__ void rope_resolve_slots(const GemvArgs& a, const int*
   }
 }
 
+// (q - z) * s of 8 codes rounded to AT, in natural k order.  fp16 scales and
+// zero points: z * s is exact in fp32, so fma(q, s, -(z * s)) is the product
+// of the exact difference rounded once; fp32 ones subtract first.
+template <int BITS, typename AT, typename ST>
+__device__ __forceinline__ u32x4 dq_exact8(uint32_t u0, uint32_t u1, float s, float z) {
+  float c[8];
+  if constexpr (BITS == 4) {
+    const uint32_t lo = u0 & 0x0F0F0F0Fu, hi = (u0 >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      c[2 * e] = (float)((lo >> (8 * e)) & 255u);
+      c[2 * e + 1] = (float)((hi >> (8 * e)) & 255u);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      c[e] = (float)((u0 >> (8 * e)) & 255u);
+      c[4 + e] = (float)((u1 >> (8 * e)) & 255u);
+    }
+  }
+  u32x4 r;
+  const float zs = -(z * s);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    float a, b;
+    if constexpr (sizeof(ST) == 2) {
+      a = fmaf(c[2 * p], s, zs);
+      b = fmaf(c[2 * p + 1], s, zs);
+    } else {
+      a = (c[2 * p] - z) * s;
+      b = (c[2 * p + 1] - z) * s;
+    }
+    r[p] = pack2<AT>(a, b);
+  }
+  return r;
+}
+
+// Epilogue of output rows nb .. nb + 3 (nb a multiple of 4) for activation
+// row m; `vec`: whole 8-byte stores apply.  One kernel serves the plain and
+// the residual product (EPI_RESIDUAL; the tests are uniform).
+template <typename AT, int EPI>
+__device__ __forceinline__ void store_out4(const GemvArgs& args, bool vec, int m, int nb, f32x4 v0, f32x4 v1) {
+  const size_t o = (size_t)m * args.N + nb;
+  if (!vec) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (nb + i >= args.N) continue;
+      if (EPI == EPI_RESIDUAL && !args.residual) store_out<AT, EPI_NONE>(args, o + i, v0[i], v1[i]);
+      else store_out<AT, EPI>(args, o + i, v0[i], v1[i]);
+    }
+    return;
+  }
+  if (nb >= args.N) return;
+  typedef AT at4 __attribute__((ext_vector_type(4)));
+  at4 a, b, c;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    a[i] = saturate_cast<AT>(v0[i]);
+    b[i] = saturate_cast<AT>(v1[i]);
+  }
+  if constexpr (EPI == EPI_RESIDUAL) {
+    if (args.y0) *reinterpret_cast<at4*>(reinterpret_cast<AT*>(args.y0) + o) = a;
+    if (!args.residual) return;
+    const at4 r = *reinterpret_cast<const at4*>(reinterpret_cast<const AT*>(args.residual) + o);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[i] = from_f32<AT>(to_f32((AT)r[i]) + to_f32((AT)a[i]));
+    *reinterpret_cast<at4*>(reinterpret_cast<AT*>(args.y1) + o) = c;
+  } else {
+    if (args.y0) *reinterpret_cast<at4*>(reinterpret_cast<AT*>(args.y0) + o) = a;
+    if (args.y1) *reinterpret_cast<at4*>(reinterpret_cast<AT*>(args.y1) + o) = b;
+    if (args.y2) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float gf = to_f32((AT)a[i]);
+        c[i] = from_f32<AT>(gf / (1.0f + expf(-gf)) * to_f32((AT)b[i]));
+      }
+      *reinterpret_cast<at4*>(reinterpret_cast<AT*>(args.y2) + o) = c;
+    }
+  }
+}
+
 // CUs of the current device, cached per device.
 inline int device_cu_count() {
   static int cache[64] = {0};
@@ -381,5 +462,14 @@ bool gemm_rows_ok(const GemvArgs& a, int64_t M, int64_t gs);
 float gemm_rows_us(int bits, int nmat, int M, int N, int K);  // estimated time of that launch
 template <int BITS, int NMAT, int EPI>
 int launch_gemm_rows(const GemvArgs& a, int act_dt, int sc_dt, hipStream_t st);
+
+// The few-row matvec (gemv_few.hip), a.M <= 32 rows (8-bit codes: 16) of what
+// few_ok accepts, with few_workspace_bytes of workspace (0 unless K is cut into
+// slices; EPI_ROPE_KV and EPI_GATE_UP need it 0).
+size_t few_workspace_bytes(int64_t M, int64_t N, int64_t K);
+template <int BITS, int NMAT>
+bool few_ok(const GemvArgs& a, int64_t M, int64_t gs, int sc_dt, size_t ws_bytes);
+template <int BITS, int NMAT, int EPI>
+int launch_few(const GemvArgs& a, int act_dt, float* ws, hipStream_t st);
 
 }  // namespace mkq

@@ -52,6 +52,9 @@ SIGNATURES: dict[str, list] = {
     "mk_quantize_weight": [_P, _P, _P, _I64, _I64, _I64, _I, _D, _I, _I, _P],
     "mk_q4_matvec": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _I, _P],
     "mk_q8_matvec": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _I, _P],
+    "mk_matvec_workspace_bytes": [_I64] * 3,
+    "mk_q4_matvec_ws": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _I, _P, _SZ, _P],
+    "mk_q8_matvec_ws": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _I, _P, _SZ, _P],
     "mk_q4_gate_up": [_P] * 10 + [_I64] * 4 + [_I, _I, _P],
     "mk_q8_gate_up": [_P] * 10 + [_I64] * 4 + [_I, _I, _P],
     "mk_argmax_rows": [_P, _P, _I64, _I64, _I, _P],
@@ -78,7 +81,7 @@ SIGNATURES: dict[str, list] = {
     "mk_paged_verify_attention": [_P] * 6 + [_I64] * 8 + [_F, _I, _P, _SZ, _P],
     "mk_paged_quantized_verify_attention": [_P] * 8 + [_I64] * 9 + [_I, _F, _I, _P, _SZ, _P],
 }
-_RESTYPES = {"mk_paged_attention_workspace_bytes": _SZ}
+_RESTYPES = {"mk_paged_attention_workspace_bytes": _SZ, "mk_matvec_workspace_bytes": _SZ}
 
 _lock = threading.Lock()
 _lib = None

@@ -271,18 +271,25 @@ def _hip_matvec(bits, x2d, w, scales, zeros, group_size, residual=None, want_mm=
     s, z = scales_for_kernel(scales, zeros)
     M, K = x2d.shape
     N = w.shape[0]
-    name = "mk_q4_matvec" if bits == 4 else "mk_q8_matvec"
+    name = "mk_q4_matvec_ws" if bits == 4 else "mk_q8_matvec_ws"
+    # fp32 sums of K slices (few rows of a long K); from the allocator, so it
+    # lives and is reused in this stream's order
+    ws, ws_bytes = None, 0
+    if M <= 64 and K > 4096:
+        ws_bytes = int(_lib.load().mk_matvec_workspace_bytes(M, N, K))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
     if residual is None:
         y = torch.empty((M, N), dtype=x2d.dtype, device=dev)
         _lib.launch(name, dev, _lib.ptr(x2d), _lib.ptr(w), _lib.ptr(s), _lib.ptr(z), None, None,
-                    _lib.ptr(y), M, N, K, group_size, _lib.dtype_code(x2d.dtype), _lib.dtype_code(s.dtype))
+                    _lib.ptr(y), M, N, K, group_size, _lib.dtype_code(x2d.dtype), _lib.dtype_code(s.dtype),
+                    _lib.ptr(ws), ws_bytes)
         return y
     residual = residual.to(x2d.dtype).contiguous()
     y_out = torch.empty((M, N), dtype=x2d.dtype, device=dev)
     y_mm = torch.empty((M, N), dtype=x2d.dtype, device=dev) if want_mm else None
     _lib.launch(name, dev, _lib.ptr(x2d), _lib.ptr(w), _lib.ptr(s), _lib.ptr(z), _lib.ptr(residual),
                 _lib.ptr(y_mm), _lib.ptr(y_out), M, N, K, group_size, _lib.dtype_code(x2d.dtype),
-                _lib.dtype_code(s.dtype))
+                _lib.dtype_code(s.dtype), _lib.ptr(ws), ws_bytes)
     return y_mm, y_out
 
 
