@@ -147,6 +147,24 @@ int mk_q8_rmsnorm_gate_up(const void* x, const void* residual, const void* norm_
                           void* up_out, void* mlp_out, int64_t M, int64_t N, int64_t K, int64_t group_size,
                           int act_dtype, int scale_dtype, int norm_w_dtype, void* stream);
 
+/* The whole MLP block (ops/mlp_block_ops.py:343-364): mk_q*_rmsnorm_gate_up
+ * (gate/up [I, K], without gate and up outputs) followed by mk_q*_matvec_ws of
+ * the down projection [K, I] with z as its residual.  z_out, normed_out [M,K]
+ * and mlp_out [M,I] receive the intermediates; the workspace is that of
+ * mk_matvec_workspace_bytes(M, K, I). */
+int mk_q4_mlp_block(const void* x, const void* residual, const void* norm_w, float eps, const uint8_t* w_gate,
+                    const uint8_t* w_up, const uint8_t* w_down, const void* s_gate, const void* s_up,
+                    const void* s_down, const void* z_gate, const void* z_up, const void* z_down, void* z_out,
+                    void* normed_out, void* mlp_out, void* out, int64_t M, int64_t I, int64_t K, int64_t group_size,
+                    int act_dtype, int scale_dtype, int down_scale_dtype, int norm_w_dtype, void* workspace,
+                    size_t workspace_bytes, void* stream);
+int mk_q8_mlp_block(const void* x, const void* residual, const void* norm_w, float eps, const uint8_t* w_gate,
+                    const uint8_t* w_up, const uint8_t* w_down, const void* s_gate, const void* s_up,
+                    const void* s_down, const void* z_gate, const void* z_up, const void* z_down, void* z_out,
+                    void* normed_out, void* mlp_out, void* out, int64_t M, int64_t I, int64_t K, int64_t group_size,
+                    int act_dtype, int scale_dtype, int down_scale_dtype, int norm_w_dtype, void* workspace,
+                    size_t workspace_bytes, void* stream);
+
 /* RMSNorm + q4/q8 matvec: y = (x * rsqrt(mean(x^2) + eps) * norm_w, rounded
  * to the activation dtype) . W^T -- the input norm and qkv projection of the
  * decode layer (ops/llama_layer_ops.py:256-260 + ops/quantized_decode_block_ops.py:

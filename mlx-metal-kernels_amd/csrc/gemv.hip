@@ -1486,6 +1486,23 @@ int norm_gate_up_entry(const void* x, const void* residual, const void* norm_w, 
                              sc_dt, stream);
 }
 
+// The whole MLP block: the front above, then down + residual z.
+template <int BITS>
+int mlp_block_entry(const void* x, const void* residual, const void* norm_w, float eps, const uint8_t* wg,
+                    const uint8_t* wu, const uint8_t* wd, const void* sg, const void* su, const void* sd,
+                    const void* zg, const void* zu, const void* zd, void* z_out, void* normed_out, void* mlp_out,
+                    void* out, int64_t M, int64_t I, int64_t K, int64_t gs, int act_dt, int sc_dt, int down_sc_dt,
+                    int nw_dt, void* ws, size_t ws_bytes, void* stream) {
+  MK_REQUIRE(wd && sd && mlp_out && out);
+  MK_REQUIRE(down_sc_dt == MK_DT_F16 || down_sc_dt == MK_DT_F32);
+  MK_REQUIRE(ws_bytes == 0 || (ws && mk_aligned(ws, 16)));
+  const int rc = norm_gate_up_entry<BITS>(x, residual, norm_w, eps, wg, wu, sg, su, zg, zu, z_out, normed_out, nullptr,
+                                          nullptr, mlp_out, M, I, K, gs, act_dt, sc_dt, nw_dt, stream);
+  if (rc != MK_OK) return rc;
+  return matvec_entry<BITS>(mlp_out, wd, sd, zd, z_out, nullptr, out, M, K, I, gs, act_dt, down_sc_dt, stream, ws,
+                            ws_bytes);
+}
+
 // RMSNorm + matvec: y = fp16(x * rsqrt(mean(x^2) + eps) * norm_w) . W^T.
 // One launch (the norm as the dot kernel's prologue, no residual) for an
 // M = 1 fp16 q4 row the dot kernel takes, else the norm kernel into
@@ -1709,6 +1726,28 @@ int mk_q8_rmsnorm_gate_up(const void* x, const void* residual, const void* norm_
   return norm_gate_up_entry<8>(x, residual, norm_w, eps, w_gate, w_up, s_gate, s_up, z_gate, z_up, z_out,
                                normed_out, gate_out, up_out, mlp_out, M, N, K, group_size, act_dtype, scale_dtype,
                                norm_w_dtype, stream);
+}
+
+int mk_q4_mlp_block(const void* x, const void* residual, const void* norm_w, float eps, const uint8_t* w_gate,
+                    const uint8_t* w_up, const uint8_t* w_down, const void* s_gate, const void* s_up,
+                    const void* s_down, const void* z_gate, const void* z_up, const void* z_down, void* z_out,
+                    void* normed_out, void* mlp_out, void* out, int64_t M, int64_t I, int64_t K, int64_t group_size,
+                    int act_dtype, int scale_dtype, int down_scale_dtype, int norm_w_dtype, void* workspace,
+                    size_t workspace_bytes, void* stream) {
+  return mlp_block_entry<4>(x, residual, norm_w, eps, w_gate, w_up, w_down, s_gate, s_up, s_down, z_gate, z_up, z_down,
+                            z_out, normed_out, mlp_out, out, M, I, K, group_size, act_dtype, scale_dtype,
+                            down_scale_dtype, norm_w_dtype, workspace, workspace_bytes, stream);
+}
+
+int mk_q8_mlp_block(const void* x, const void* residual, const void* norm_w, float eps, const uint8_t* w_gate,
+                    const uint8_t* w_up, const uint8_t* w_down, const void* s_gate, const void* s_up,
+                    const void* s_down, const void* z_gate, const void* z_up, const void* z_down, void* z_out,
+                    void* normed_out, void* mlp_out, void* out, int64_t M, int64_t I, int64_t K, int64_t group_size,
+                    int act_dtype, int scale_dtype, int down_scale_dtype, int norm_w_dtype, void* workspace,
+                    size_t workspace_bytes, void* stream) {
+  return mlp_block_entry<8>(x, residual, norm_w, eps, w_gate, w_up, w_down, s_gate, s_up, s_down, z_gate, z_up, z_down,
+                            z_out, normed_out, mlp_out, out, M, I, K, group_size, act_dtype, scale_dtype,
+                            down_scale_dtype, norm_w_dtype, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

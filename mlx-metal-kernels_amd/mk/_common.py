@@ -31,9 +31,14 @@ def scales_for_kernel(scales: torch.Tensor, zeros: torch.Tensor | None):
     kernel boundary, ops/quant_ops.py:424)."""
     use_f16 = scales.dtype == torch.float16 and (zeros is None or zeros.dtype == torch.float16)
     target = torch.float16 if use_f16 else torch.float32
-    s = scales.to(target).contiguous()
-    z = None if zeros is None else zeros.to(target).contiguous()
-    return s, z
+    return as_dense(scales, target), as_dense(zeros, target)
+
+
+def as_dense(t, dtype):
+    """``t`` contiguous and in ``dtype`` (itself when it is; None stays None)."""
+    if t is None or (t.dtype == dtype and t.is_contiguous()):
+        return t
+    return t.to(dtype).contiguous()
 
 
 def as_u8(t: torch.Tensor) -> torch.Tensor:

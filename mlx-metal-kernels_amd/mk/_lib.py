@@ -64,6 +64,8 @@ SIGNATURES: dict[str, list] = {
     "mk_q8_rmsnorm_matvec": [_P, _P, _F] + [_P] * 5 + [_I64] * 4 + [_I, _I, _I, _P],
     "mk_q4_rmsnorm_gate_up": [_P, _P, _P, _F] + [_P] * 11 + [_I64] * 4 + [_I, _I, _I, _P],
     "mk_q8_rmsnorm_gate_up": [_P, _P, _P, _F] + [_P] * 11 + [_I64] * 4 + [_I, _I, _I, _P],
+    "mk_q4_mlp_block": [_P, _P, _P, _F] + [_P] * 13 + [_I64] * 4 + [_I, _I, _I, _I, _P, _SZ, _P],
+    "mk_q8_mlp_block": [_P, _P, _P, _F] + [_P] * 13 + [_I64] * 4 + [_I, _I, _I, _I, _P, _SZ, _P],
     "mk_swiglu": [_P, _P, _P, _I64, _I, _P],
     "mk_residual_add": [_P, _P, _P, _I64, _I, _P],
     "mk_rms_norm": [_P, _P, _P, _I64, _I64, _F, _I, _I, _P],
@@ -159,27 +161,43 @@ def require_device(*tensors) -> torch.device:
             continue
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"expected a torch.Tensor, got {type(t).__name__}")
-        if t.device.type != "cuda":
+        d = t.device
+        if d == dev:
+            continue
+        if d.type != "cuda":
             raise ValueError(
-                f"HIP backends need tensors on a ROCm device, got a tensor on {t.device}; "
+                f"HIP backends need tensors on a ROCm device, got a tensor on {d}; "
                 "use backend='reference' for host tensors"
             )
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError(f"tensors are on different devices: {dev} and {t.device}")
+        if dev is not None:
+            raise ValueError(f"tensors are on different devices: {dev} and {d}")
+        dev = d
     if dev is None:
         raise ValueError("no device tensor given")
     return dev
 
 
+def raw_stream(device: torch.device) -> int:
+    """The current stream of ``device`` as an integer handle (no Stream object
+    is made: that costs 2 us a call)."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+# what torch.cuda.current_stream / current_device wrap, where torch has them
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def launch(name: str, device: torch.device, *args) -> int:
     """Call ``name`` with ``args`` on the current stream of ``device``."""
-    lib = load()
-    fn = getattr(lib, name)
-    with torch.cuda.device(device):
-        stream = torch.cuda.current_stream(device).cuda_stream
-        rc = fn(*args, ctypes.c_void_p(stream))
+    fn = getattr(_lib if _lib is not None else load(), name)
+    if _get_device is not None and torch.cuda.is_initialized() and device.index == _get_device():
+        rc = fn(*args, raw_stream(device))
+    else:
+        with torch.cuda.device(device):
+            rc = fn(*args, torch.cuda.current_stream(device).cuda_stream)
     if rc != MK_OK:
         if rc == MK_ERR_INVALID:
             raise RuntimeError(f"{name}: invalid argument (status {rc})")
@@ -214,7 +232,7 @@ _WS_LOCK = threading.Lock()
 def _stream_workspace(kind: str, device: torch.device, nbytes: int):
     size = (nbytes + 255) // 256 * 256
     dev = torch.device(device)
-    key = (kind, dev.index, torch.cuda.current_stream(dev).cuda_stream)
+    key = (kind, dev.index, raw_stream(dev))
     capturing = torch.cuda.is_current_stream_capturing()
     with _WS_LOCK:
         buf = _WORKSPACES.get(key)

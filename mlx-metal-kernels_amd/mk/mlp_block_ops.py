@@ -12,11 +12,15 @@ are unchanged:
        (mk_q{4,8}_rmsnorm_gate_up: one kernel for an fp16 decode row, the
        norm kernel then the gate/up kernel otherwise)
     2. down matvec, residual epilogue     (mk_q{4,8}_matvec with residual)
+both made by one call of the library (mk_q{4,8}_mlp_block) unless the
+intermediates are asked for.
 """
 
 from __future__ import annotations
 
 import math
+
+import torch
 
 from .activation_ops import fused_swiglu, reference_swiglu, swiglu
 from .fused_ops import reference_residual_add, residual_add
@@ -30,8 +34,10 @@ from .quant_ops import (
     q_rmsnorm_gate_up_swiglu,
     reference_q4_matvec_decode,
     reference_q8_matvec_decode,
+    _validate_gate_up_shapes,
 )
-from ._common import ci_safe_mode_enabled
+from . import _lib
+from ._common import as_dense, as_u8, ci_safe_mode_enabled, scales_for_kernel
 
 
 def _validate_bits(bits: int) -> int:
@@ -66,7 +72,10 @@ def _validate_quantized_linear_shapes(x2d, w, scales, zeros, *, bits, group_size
         raise ValueError(f"{name} input must normalize to [rows,K], got {tuple(x2d.shape)}")
     if w.ndim != 2:
         raise ValueError(f"{name} weights must be 2-D, got {tuple(w.shape)}")
-    in_dim = x2d.shape[1]
+    return _validate_linear_weights(x2d.shape[1], w, scales, zeros, bits, group_size, name)
+
+
+def _validate_linear_weights(in_dim, w, scales, zeros, bits, group_size, name):
     out_dim = w.shape[0]
     if bits == 4:
         expected_cols = math.ceil(in_dim / 2)
@@ -176,6 +185,49 @@ def _all_hip(norm_backend, matvec_backend, activation_backend, residual_backend)
     )
 
 
+def _hip_mlp_block(x, residual, norm_weight, gate_w, up_w, down_w, gate_scales, up_scales, down_scales, gate_zeros,
+                   up_zeros, down_zeros, bits, group_size, eps):
+    """q_rmsnorm_gate_up_swiglu and q_matvec_residual in one call of the
+    library, with the intermediates in one scratch buffer.  At decode sizes the
+    host's work bounds the block (one row: 53 us of host for 24 us of kernels as
+    two calls with a tensor for each intermediate)."""
+    rows, k_dim = x.shape[0] * x.shape[1], x.shape[2]
+    x2d = x.reshape(rows, k_dim)
+    _, _, out_dim = _validate_gate_up_shapes(x2d, gate_w, up_w, gate_scales, up_scales, gate_zeros, up_zeros,
+                                             bits=bits, group_size=group_size)
+    x2d = x2d.contiguous()
+    r2d = as_dense(residual, x2d.dtype)
+    nw = norm_weight.contiguous()
+    gw, uw = as_u8(gate_w), as_u8(up_w)
+    _lib.require_device(x2d, r2d, nw, gw, uw, gate_scales, up_scales, gate_zeros, up_zeros)
+    _validate_linear_weights(out_dim, down_w, down_scales, down_zeros, bits, group_size, "quantized_linear")
+    dw = as_u8(down_w)
+    dev = _lib.require_device(x2d, dw, down_scales, down_zeros)
+    f16 = torch.float16
+    all_f16 = (gate_scales.dtype == f16 and up_scales.dtype == f16 and (gate_zeros is None or gate_zeros.dtype == f16)
+               and (up_zeros is None or up_zeros.dtype == f16))
+    tgt = f16 if all_f16 else torch.float32
+    sg, su = as_dense(gate_scales, tgt), as_dense(up_scales, tgt)
+    zg, zu = as_dense(gate_zeros, tgt), as_dense(up_zeros, tgt)
+    sd, zd = scales_for_kernel(down_scales, down_zeros)
+    # the down projection's workspace, then z and normed [rows, D] and the
+    # hidden activations [rows, I], each from a 256-byte boundary
+    ws_b = 0
+    if rows <= 64 and out_dim > 4096:
+        ws_b = (_lib.load().mk_matvec_workspace_bytes(rows, k_dim, out_dim) + 255) & -256
+    row_b = (2 * rows * k_dim + 255) & -256
+    scratch = torch.empty(ws_b + 2 * row_b + 2 * rows * out_dim, dtype=torch.uint8, device=dev)
+    out = torch.empty((rows, k_dim), dtype=x2d.dtype, device=dev)
+    ws = scratch.data_ptr()
+    z = ws + ws_b
+    _lib.launch("mk_q4_mlp_block" if bits == 4 else "mk_q8_mlp_block", dev, x2d.data_ptr(), r2d.data_ptr(),
+                nw.data_ptr(), float(eps), gw.data_ptr(), uw.data_ptr(), dw.data_ptr(), sg.data_ptr(), su.data_ptr(),
+                sd.data_ptr(), _lib.ptr(zg), _lib.ptr(zu), _lib.ptr(zd), z, z + row_b, z + 2 * row_b, out.data_ptr(),
+                rows, out_dim, k_dim, group_size, _lib.dtype_code(x2d.dtype), _lib.dtype_code(tgt),
+                _lib.dtype_code(sd.dtype), _lib.dtype_code(nw.dtype), ws if ws_b else None, ws_b)
+    return out.reshape(x.shape)
+
+
 def quantized_mlp_block(x, residual, norm_weight, gate_w, gate_scales, up_w, up_scales, down_w, down_scales, *,
                         gate_zeros=None, up_zeros=None, down_zeros=None, bits=4, group_size=32, eps=1e-5,
                         backend_preset=None, norm_backend="metal", matvec_backend="metal_tiled",
@@ -195,6 +247,9 @@ def quantized_mlp_block(x, residual, norm_weight, gate_w, gate_scales, up_w, up_
     if _all_hip(norm_backend, matvec_backend, activation_backend, residual_backend):
         _validate_bits(bits)
         gate = up = None
+        if not return_intermediates and x.numel() and down_w.ndim == 2 and down_w.shape[0] == x.shape[2]:
+            return _hip_mlp_block(x, residual, norm_weight, gate_w, up_w, down_w, gate_scales, up_scales, down_scales,
+                                  gate_zeros, up_zeros, down_zeros, bits, group_size, eps)
         if return_intermediates:
             z, normed, gate, up, mlp = q_rmsnorm_gate_up_swiglu(
                 x, residual, norm_weight, gate_w, up_w, gate_scales, up_scales, gate_zeros, up_zeros, bits=bits,

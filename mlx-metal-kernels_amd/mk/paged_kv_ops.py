@@ -21,7 +21,7 @@ import os
 import torch
 
 from . import _lib
-from ._common import ACT_DTYPES, ci_safe_mode_enabled
+from ._common import ACT_DTYPES, as_dense, ci_safe_mode_enabled
 from .kv_cache_ops import _normalize_token_shape, normalize_positions
 
 _ATTN_BACKENDS_MSG = "backend must be one of 'reference', 'metal', 'metal_threadgroup', 'metal_d64', 'metal_d128', 'auto'"
@@ -86,6 +86,8 @@ def _validate_page_tensors(K_pages, V_pages, block_table):
 
 
 def _i32(t: torch.Tensor, device) -> torch.Tensor:
+    if t.dtype == torch.int32 and t.device == device and t.is_contiguous():
+        return t
     return t.to(device=device, dtype=torch.int32).contiguous()
 
 
@@ -246,7 +248,7 @@ def _hip_paged_attention(q3, K_pages, V_pages, block_table, lengths, scale: floa
     dtype = K_pages.dtype
     if V_pages.dtype != dtype:
         raise TypeError(f"K_pages and V_pages must share a dtype, got {dtype}, {V_pages.dtype}")
-    q3 = q3.to(dtype).contiguous()
+    q3 = as_dense(q3, dtype)
     Kp, Vp = K_pages.contiguous(), V_pages.contiguous()
     bt = _i32(block_table, dev)
     ln = _i32(lengths, dev)

@@ -23,7 +23,7 @@ import os
 import torch
 
 from . import _lib
-from ._common import ACT_DTYPES, as_u8, ci_safe_mode_enabled, finfo_max, scales_for_kernel
+from ._common import ACT_DTYPES, as_dense, as_u8, ci_safe_mode_enabled, finfo_max, scales_for_kernel
 
 _MATVEC_BACKENDS_MSG = "backend must be one of 'reference', 'metal', 'metal_parallel', 'metal_tiled', 'auto'"
 
@@ -284,7 +284,7 @@ def _hip_matvec(bits, x2d, w, scales, zeros, group_size, residual=None, want_mm=
                     _lib.ptr(y), M, N, K, group_size, _lib.dtype_code(x2d.dtype), _lib.dtype_code(s.dtype),
                     _lib.ptr(ws), ws_bytes)
         return y
-    residual = residual.to(x2d.dtype).contiguous()
+    residual = as_dense(residual, x2d.dtype)
     y_out = torch.empty((M, N), dtype=x2d.dtype, device=dev)
     y_mm = torch.empty((M, N), dtype=x2d.dtype, device=dev) if want_mm else None
     _lib.launch(name, dev, _lib.ptr(x2d), _lib.ptr(w), _lib.ptr(s), _lib.ptr(z), _lib.ptr(residual),
@@ -381,11 +381,7 @@ def _hip_gate_up(bits, x, gate_w, up_w, gate_scales, up_scales, gate_zeros, up_z
     # both streams share one scale dtype
     all_f16 = all(t is None or t.dtype == torch.float16 for t in (gate_scales, up_scales, gate_zeros, up_zeros))
     tgt = torch.float16 if all_f16 else torch.float32
-
-    def cvt(t):
-        return None if t is None else t.to(tgt).contiguous()
-
-    sg, su, zg, zu = cvt(gate_scales), cvt(up_scales), cvt(gate_zeros), cvt(up_zeros)
+    sg, su, zg, zu = (as_dense(t, tgt) for t in (gate_scales, up_scales, gate_zeros, up_zeros))
     outs = []
     gate = torch.empty((rows, out_dim), dtype=x2d.dtype, device=dev) if want_gate else None
     up = torch.empty((rows, out_dim), dtype=x2d.dtype, device=dev) if want_up else None
@@ -438,11 +434,7 @@ def q_rmsnorm_gate_up_swiglu(x, residual, norm_weight, gate_w, up_w, gate_scales
     dev = _lib.require_device(x2d, r2d, nw, gw, uw, gate_scales, up_scales, gate_zeros, up_zeros)
     all_f16 = all(t is None or t.dtype == torch.float16 for t in (gate_scales, up_scales, gate_zeros, up_zeros))
     tgt = torch.float16 if all_f16 else torch.float32
-
-    def cvt(t):
-        return None if t is None else t.to(tgt).contiguous()
-
-    sg, su, zg, zu = cvt(gate_scales), cvt(up_scales), cvt(gate_zeros), cvt(up_zeros)
+    sg, su, zg, zu = (as_dense(t, tgt) for t in (gate_scales, up_scales, gate_zeros, up_zeros))
     z = torch.empty_like(x2d)
     normed = torch.empty_like(x2d)
     gate = torch.empty((rows, out_dim), dtype=x2d.dtype, device=dev) if return_gate_up else None
