@@ -275,7 +275,7 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2)
     // SZ8: the group of this lane's 16 k (past K: the row's last one)
     const int grp = min(((st0 + it) * GK + 16 * kb) >> args.lg, G - 1);
     codes_t c[GNT];
-    float sf[GNT], zf[GNT];
+    ExactGp<ST> ge[GNT];
     GpNat gp[GNT];
 #pragma unroll
     for (int t = 0; t < GNT; ++t) {
@@ -292,14 +292,13 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2)
       if constexpr (MAGIC) {
         gp[t] = make_gp_nat<BITS>((f16)sv, (f16)zv);
       } else {
-        sf[t] = to_f32(sv);
-        zf[t] = to_f32(zv);
+        ge[t] = make_exact_gp<ST>(sv, zv);
       }
     }
     auto dequant = [&](int t, int h) {
       const uint32_t u0 = c[t][BITS == 4 ? h : 2 * h], u1 = c[t][BITS == 4 ? h : 2 * h + 1];
       if constexpr (MAGIC) return dq_nat8<BITS>(u0, u1, gp[t], magic);
-      else return dq_exact8<BITS, AT, ST>(u0, u1, sf[t], zf[t]);
+      else return dq_exact8<BITS, AT, ST>(u0, u1, ge[t]);
     };
     // Chunks of two column tiles: a chunk requests the next one's activation
     // operands and unpacks a part of the second half's weights beside its

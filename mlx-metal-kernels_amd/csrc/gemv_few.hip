@@ -21,8 +21,8 @@
 // 4096 x 14336 + residual | 6144 x 4096 | 4096 x 4096, g64, q8 g32):
 //   q4 fp16  8 rows  22.7 -> 20.6 | 18.4 -> 16.7 | 10.8 -> 8.6 | 8.0 -> 6.4
 //   q4 fp16 32 rows  30.1 -> 23.6 | 35.3 -> 22.2 | 16.9 -> 12.2 | 13.7 -> 9.8
-//   q4 bf16  4 rows  36.1 -> 27.7 | 21.2 -> 19.9 | 12.7 -> 10.8 | 9.1 -> 7.4
-//   q4 bf16 32 rows  78.8 -> 34.2 | 52.9 -> 29.8 | 32.2 -> 14.3 | 19.7 -> 10.5
+//   q4 bf16  4 rows  36.1 -> 26.1 | 21.2 -> 17.2 | 12.7 ->  9.2 | 9.1 -> 6.0
+//   q4 bf16 32 rows  78.8 -> 29.7 | 52.9 -> 25.1 | 32.2 -> 12.2 | 19.7 -> 9.0
 //   q8 fp16  8 rows  46.4 -> 34.3 | 28.3 -> 20.6 | 16.3 -> 11.2 | 10.2 -> 8.3
 // What is left is the stream: 128256 x 4096 at 8 rows takes 68 us (78 before),
 // 60 without the unpacking and products, 65 without the turns' barriers.
@@ -263,23 +263,22 @@ __global__ __launch_bounds__(64 * FMAXW) __attribute__((amdgpu_waves_per_eu(XL ?
     sz_at<BITS, LG>(sz[u], j, kb, &sv, &zv);
     if (!has_z) zv = (f16)0.0f;
     GpMagic gp;
-    float sf = 0.0f, zf = 0.0f;
+    ExactGp<f16> ge;
     if constexpr (MAGIC) {
       gp = make_gp_magic(sv, zv);
     } else {
-      sf = to_f32(sv);
-      zf = to_f32(zv);
+      ge = make_exact_gp<f16>(sv, zv);
     }
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
       u32x4 a;
       if constexpr (BITS == 4) {
         if constexpr (MAGIC) a = dq4_magic(w[u][j][0][st], gp, magic, magic_hi);
-        else a = dq_exact8<4, AT, f16>(w[u][j][0][st], 0u, sf, zf);
+        else a = dq_exact8<4, AT, f16>(w[u][j][0][st], 0u, ge);
       } else {
         const uint32_t u0 = w[u][j][st >> 1][(2 * st) & 3], u1 = w[u][j][st >> 1][(2 * st + 1) & 3];
         if constexpr (MAGIC) a = dq8_magic(u0, u1, gp, magic);
-        else a = dq_exact8<8, AT, f16>(u0, u1, sf, zf);
+        else a = dq_exact8<8, AT, f16>(u0, u1, ge);
       }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma_k32<AT>(a, xp[mt][x0 + st], acc[mt]);
@@ -430,8 +429,8 @@ int few_columns(const GemvArgs& a, float* ws, hipStream_t st) {
   const int run = (p.tiles + p.runs - 1) / p.runs;  // tiles of the longest run
   // Up to 8 rows of the forms whose unpacking weighs most, while tiles are
   // few: one tile per workgroup (XL), two workgroups a CU.  Against the ring,
-  // us at 8 rows: bf16 q4 2 x 14336 x 4096 28.5 / 31.8, 4096 x 14336 21.0 /
-  // 22.2; q8 g32 fp16 6144 x 4096 11.2 / 14.1, 4096 x 4096 8.3 / 9.3.  The ring
+  // us: bf16 q4 MLP block of 4096 and 14336 44.4 / 47.9 at 4 rows, 47.3 / 48.7
+  // at 8, 4096 x 14336 17.0 / 18.8 at 4; at 8 rows q8 g32 fp16 6144 x 4096 11.2 / 14.1, 4096 x 4096 8.3 / 9.3.  The ring
   // is ahead for fp16 q4 (16.7 / 17.6 at 4096 x 14336), for q8 pairs (34.3 /
   // 45.4) and where tiles are many (fp16 q4 128256 x 4096 68 / 96).
   constexpr bool ONE = NMAT == 2 ? BITS == 4 && !__is_same(AT, f16) : BITS == 8 || !__is_same(AT, f16);
