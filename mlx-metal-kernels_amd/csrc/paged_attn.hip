@@ -209,22 +209,26 @@ __device__ __forceinline__ u32x4 deq8x8(uint32_t u0, uint32_t u1, f16x2 s2) {
   r[3] = q8_pair(u1, 8, s2);
   return r;
 }
+// 1024.0h and 64.0h in vector registers: with the mask in a scalar one, mask
+// and magic are one v_and_or_b32 (as literals they are two instructions)
+struct Q4Magic {
+  uint32_t lo, hi;
+};
+__device__ __forceinline__ Q4Magic q4_magic() { return {in_vgpr(0x64006400u), in_vgpr(0x54005400u)}; }
 // 8 q4 codes (one word) -> 8 fp16, order [0,4,1,5,2,6,3,7].  Even nibbles
 // sit at mantissa bits 0..3 of 1024.0h (ulp 1): 1024 + c.  Odd nibbles stay
 // in place at bits 4..7 under the exponent of 64.0h (ulp 1/16): 64 + c.  So
 // both halves give (c - 8) exactly after one subtraction and share the same
 // scale multiply, which rounds (c - 8) * s once -- one shift per word.
-__device__ __forceinline__ u32x4 deq4x8(uint32_t u, f16x2 s2) {
+__device__ __forceinline__ u32x4 deq4x8(uint32_t u, f16x2 s2, Q4Magic mg) {
   const f16x2 k_lo = {(f16)1032.0f, (f16)1032.0f};  // 1024 + 8
   const f16x2 k_hi = {(f16)72.0f, (f16)72.0f};      // 64 + 8
-  const uint32_t magic_lo = 0x64006400u;            // 1024.0h
-  const uint32_t magic_hi = 0x54005400u;            // 64.0h
   const uint32_t v = u >> 8;
   u32x4 r;
-  r[0] = bitcast<uint32_t>((bitcast<f16x2>((u & 0x000F000Fu) | magic_lo) - k_lo) * s2);
-  r[1] = bitcast<uint32_t>((bitcast<f16x2>((u & 0x00F000F0u) | magic_hi) - k_hi) * s2);
-  r[2] = bitcast<uint32_t>((bitcast<f16x2>((v & 0x000F000Fu) | magic_lo) - k_lo) * s2);
-  r[3] = bitcast<uint32_t>((bitcast<f16x2>((v & 0x00F000F0u) | magic_hi) - k_hi) * s2);
+  r[0] = bitcast<uint32_t>((bitcast<f16x2>((u & 0x000F000Fu) | mg.lo) - k_lo) * s2);
+  r[1] = bitcast<uint32_t>((bitcast<f16x2>((u & 0x00F000F0u) | mg.hi) - k_hi) * s2);
+  r[2] = bitcast<uint32_t>((bitcast<f16x2>((v & 0x000F000Fu) | mg.lo) - k_lo) * s2);
+  r[3] = bitcast<uint32_t>((bitcast<f16x2>((v & 0x00F000F0u) | mg.hi) - k_hi) * s2);
   return r;
 }
 
@@ -246,6 +250,14 @@ __device__ __forceinline__ u32x4 deq4x8(uint32_t u, f16x2 s2) {
 // consumed.  Loads are branch-free -- positions past the split's end or on
 // an unmapped page read a clamped in-bounds row and are masked out of the
 // softmax (their V is zeroed) -- so the compiler's wait counts stay exact.
+// Quantized caches are bound by the vector ALU (q4: 75 % of its cycles issue),
+// so what every lane would compute alike is kept in scalar registers: the wave
+// index and a pair's block count are made scalar, and with them page rows,
+// bases and branches.  Per block and wave 531 -> about 400 vector instructions
+// with q4's and-or unpacking, us per call (32 / 8 heads of 128): q4 8 x 32768
+// positions 94.4 -> 80.4, 32 x 8192 76.8 -> 64.2; q8 8 x 32768 116 -> 109; fp16
+// (bound by the pages' stream) unchanged.  A third block buffer for q4, 2 blocks
+// ahead, gains nothing (94.9 before, 82.9 after).
 // Page ids of the split are read once (see SplitCtx).  Splits that do not
 // finish their sequence write (m, l, O) partials that paged_attn_merge_kernel
 // combines.
@@ -311,14 +323,14 @@ __device__ __forceinline__ u32x4 qperm(u32x4 X) {
 __device__ __forceinline__ u32x2 deq8x4(uint32_t u, f16x2 s2) {
   return (u32x2){q8_pair(u, 0, s2), q8_pair(u, 8, s2)};
 }
-__device__ __forceinline__ u32x2 deq4x4(uint32_t u, f16x2 s2) {
+__device__ __forceinline__ u32x2 deq4x4(uint32_t u, f16x2 s2, Q4Magic mg) {
   // bytes (b0, 0, b1, 0): n0 n1 @ bits 0..7, n2 n3 @ 16..23, one v_perm_b32;
   // the odd nibbles stay in place under 64.0h as in deq4x8
   const uint32_t t = perm_b32(0u, u, 0x04010400u);
   const f16x2 k_lo = {(f16)1032.0f, (f16)1032.0f};
   const f16x2 k_hi = {(f16)72.0f, (f16)72.0f};
-  return (u32x2){bitcast<uint32_t>((bitcast<f16x2>((t & 0x000F000Fu) | 0x64006400u) - k_lo) * s2),
-                 bitcast<uint32_t>((bitcast<f16x2>((t & 0x00F000F0u) | 0x54005400u) - k_hi) * s2)};
+  return (u32x2){bitcast<uint32_t>((bitcast<f16x2>((t & 0x000F000Fu) | mg.lo) - k_lo) * s2),
+                 bitcast<uint32_t>((bitcast<f16x2>((t & 0x00F000F0u) | mg.hi) - k_hi) * s2)};
 }
 
 __device__ __forceinline__ f16x2 splat_h(uint32_t s) {
@@ -671,8 +683,8 @@ struct LaneOffsets {
   uint32_t k0;                     // K codes of run 0 of row r16
   uint32_t v0;                     // V chunk of row 4kb
   uint32_t rs;                     // bytes between positions of a page (wave-uniform)
-  uint32_t ks[NKS > 0 ? NKS : 1];  // K scale (elements) of the lane's chunks
-  uint32_t vs[4];                  // V scale (elements)
+  uint32_t ks[NKS > 0 ? NKS : 1];  // K scales of the lane's chunks
+  uint32_t vs[4];                  // V scales
 };
 
 // The lane offsets of the PT addressing mode for lane (r16, kb).
@@ -689,23 +701,33 @@ __device__ __forceinline__ LaneOffsets<KVF, D, SB> pt_lane_offsets(const PagedAr
 #pragma unroll
     for (int e = 0; e < KVBlock<KVF, D, SB>::NKS; ++e) {
       const int j = SB ? e * F::KRUN : e;
-      lo.ks[e] = (uint32_t)r16 * ss + (uint32_t)(F::dbase(j, kb) >> a.lg_gs);
+      lo.ks[e] = 2u * ((uint32_t)r16 * ss + (uint32_t)(F::dbase(j, kb) >> a.lg_gs));
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) lo.vs[i] = (uint32_t)(4 * kb + i) * ss + (uint32_t)((r16 * F::DPL) >> a.lg_gs);
+    for (int i = 0; i < 4; ++i) lo.vs[i] = 2u * ((uint32_t)(4 * kb + i) * ss + (uint32_t)((r16 * F::DPL) >> a.lg_gs));
   }
   return lo;
 }
 
 template <typename AT, int D, int KVF, bool SB, bool PT>
 __device__ __forceinline__ void load_block(KVBlock<KVF, D, SB>& blk, const PagedArgs& a,
-                                           const SplitCtx& c, const LaneOffsets<KVF, D, SB>& lo,
+                                           const SplitCtx& c, LaneOffsets<KVF, D, SB>& lo,
                                            int tb, int r16, int kb) {
   using F = Fmt<KVF, D>;
   constexpr int NKS = KVBlock<KVF, D, SB>::NKS;
   const uint8_t* Kb = reinterpret_cast<const uint8_t*>(a.K);
   const uint8_t* Vb = reinterpret_cast<const uint8_t*>(a.V);
   if constexpr (PT) {
+    // scalar base + 32-bit lane offset is an addressing mode, taken only where
+    // the offset is seen to be 32 bits wide (widened once before the loop, every
+    // load has a 64-bit addition)
+    asm volatile("" : "+v"(lo.k0), "+v"(lo.v0));
+    if constexpr (KVF != 0) {
+#pragma unroll
+      for (int e = 0; e < NKS; ++e) asm volatile("" : "+v"(lo.ks[e]));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(lo.vs[i]));
+    }
     uint32_t m = 0;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -740,12 +762,12 @@ __device__ __forceinline__ void load_block(KVBlock<KVF, D, SB>& blk, const Paged
         blk.v[4 * u + i] = x;
       }
       if constexpr (KVF != 0) {
-        const uint16_t* kst = a.Ks + (uint64_t)row0 * a.ngroups;
-        const uint16_t* vst = a.Vs + (uint64_t)row0 * a.ngroups;
+        const uint8_t* kst = reinterpret_cast<const uint8_t*>(a.Ks + (uint64_t)row0 * a.ngroups);
+        const uint8_t* vst = reinterpret_cast<const uint8_t*>(a.Vs + (uint64_t)row0 * a.ngroups);
 #pragma unroll
-        for (int e = 0; e < NKS; ++e) blk.ks[u][e] = kst[lo.ks[e]];
+        for (int e = 0; e < NKS; ++e) blk.ks[u][e] = *reinterpret_cast<const uint16_t*>(kst + lo.ks[e]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) blk.vs[4 * u + i] = vst[lo.vs[i]];
+        for (int i = 0; i < 4; ++i) blk.vs[4 * u + i] = *reinterpret_cast<const uint16_t*>(vst + lo.vs[i]);
       }
     }
     blk.mask = m;
@@ -804,7 +826,7 @@ __device__ __forceinline__ void load_block(KVBlock<KVF, D, SB>& blk, const Paged
 
 // 8 act-type values of K step j (order as qperm<KVF>)
 template <typename AT, int D, int KVF, bool SB>
-__device__ __forceinline__ u32x4 k_operand(const KVBlock<KVF, D, SB>& blk, int u, int j) {
+__device__ __forceinline__ u32x4 k_operand(const KVBlock<KVF, D, SB>& blk, int u, int j, Q4Magic mg) {
   using F = Fmt<KVF, D>;
   const int r = j / F::KRUN, e = j % F::KRUN;
   if constexpr (KVF == 0) {
@@ -812,22 +834,22 @@ __device__ __forceinline__ u32x4 k_operand(const KVBlock<KVF, D, SB>& blk, int u
   } else {
     const f16x2 s2 = splat_h(blk.ks[u][SB ? r : j]);
     if constexpr (KVF == 8) return deq8x8(blk.k[u][r][2 * e], blk.k[u][r][2 * e + 1], s2);
-    else return deq4x8(blk.k[u][r][e], s2);
+    else return deq4x8(blk.k[u][r][e], s2, mg);
   }
 }
 
 // V chunk of position p as DPL act-type values in slot order (Fmt::vslot)
 template <int D, int KVF, bool SB>
-__device__ __forceinline__ u32x4 v_chunk(const KVBlock<KVF, D, SB>& blk, int p) {
+__device__ __forceinline__ u32x4 v_chunk(const KVBlock<KVF, D, SB>& blk, int p, Q4Magic mg) {
   if constexpr (KVF == 0) {
     return blk.v[p];
   } else {
     const f16x2 s2 = splat_h(blk.vs[p]);
     if constexpr (D == 128) {
       if constexpr (KVF == 8) return deq8x8(blk.v[p][0], blk.v[p][1], s2);
-      else return deq4x8(blk.v[p][0], s2);
+      else return deq4x8(blk.v[p][0], s2, mg);
     } else {
-      const u32x2 x = KVF == 8 ? deq8x4(blk.v[p][0], s2) : deq4x4(blk.v[p][0], s2);
+      const u32x2 x = KVF == 8 ? deq8x4(blk.v[p][0], s2) : deq4x4(blk.v[p][0], s2, mg);
       return (u32x4){x[0], x[1], 0u, 0u};
     }
   }
@@ -964,13 +986,14 @@ __device__ __forceinline__ void consume_block(const KVBlock<KVF, D, SB> blk,
                                               float& l_run, f32x4 (&o)[Fmt<KVF, D>::DPL]) {
   constexpr int KSTEPS = Fmt<KVF, D>::KSTEPS;
   constexpr int DPL = Fmt<KVF, D>::DPL;
+  const Q4Magic mg = KVF == 4 ? q4_magic() : Q4Magic{0u, 0u};
   // ---- S^T = K q^T for the two 16-position tiles
   f32x4 sc[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < KSTEPS; ++j) acc = mfma_k32<AT>(k_operand<AT, D, KVF, SB>(blk, u, j), qv[j], acc);
+    for (int j = 0; j < KSTEPS; ++j) acc = mfma_k32<AT>(k_operand<AT, D, KVF, SB>(blk, u, j, mg), qv[j], acc);
     sc[u] = acc;
   }
   // ---- scores (base 2); lane holds S[16u + 4kb + i][head r16]
@@ -1039,7 +1062,7 @@ __device__ __forceinline__ void consume_block(const KVBlock<KVF, D, SB> blk,
   // cache contents cannot reach the output through p = 0
   u32x4 vc[8];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) vc[q] = v_chunk<D, KVF, SB>(blk, q);
+  for (int q = 0; q < 8; ++q) vc[q] = v_chunk<D, KVF, SB>(blk, q, mg);
   if (!full) {
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
@@ -1074,6 +1097,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   const int lane = threadIdx.x & 63;
   const int r16 = lane & 15;
   const int kb = lane >> 4;
+  // (a scalar: the kv head, and with it every page address, stays in scalar
+  // registers)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // workgroup -> (pair, group of wg_units units); wave -> unit = (kv head,
   // block of 16 query heads).  The units of a pair read the same pages (one
   // kv head's slice of every position each), so they share a workgroup: the
@@ -1084,7 +1110,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   // spreads every head over all XCDs.
   const int groups = a.units / a.wg_units;
   const int pair = (int)blockIdx.x / groups;
-  const int unit = (((int)blockIdx.x - pair * groups) * a.wg_units + (int)(threadIdx.x >> 6) +
+  const int unit = (((int)blockIdx.x - pair * groups) * a.wg_units + wave +
                     (a.wg_units == 1 ? pair : 0)) % a.units;
   const int hkv = unit / a.HB;
   const int hb = unit - hkv * a.HB;
@@ -1098,7 +1124,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   // (segments 1 .. kQSlots-1): kMaxSegs descriptors (a pair holds at most
   // cap_blk <= 64 blocks, so at most 64 segments)
   extern __shared__ __align__(16) uint8_t attn_dyn[];
-  u32x4* qslots = reinterpret_cast<u32x4*>(attn_dyn + (size_t)(threadIdx.x >> 6) * attn_wave_lds<D>());
+  u32x4* qslots = reinterpret_cast<u32x4*>(attn_dyn + (size_t)wave * attn_wave_lds<D>());
   SegDesc* sd = reinterpret_cast<SegDesc*>(qslots + (kQSlots - 1) * KSTEPS * 64);
   int* slen = reinterpret_cast<int*>(sd + kMaxSegs);  // verify: segment s's sequence length
   const VRows vr = VW ? vrows(a, h0) : VRows{0, 0};
@@ -1176,7 +1202,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   // the end reloads the last block, masked off.  Loads run one block ahead of
   // the consumes and cross segment boundaries: the load side (c, segL) and the
   // consume side (segC) each step to the next segment when they reach it.
-  const int nbt = (int)(g1 - g0);
+  const int nbt = __builtin_amdgcn_readfirstlane((int)(g1 - g0));  // wave-uniform (the plan is in vector registers)
   Blk A, Bq;
 #pragma unroll
   for (int u = 0; u < 2; ++u)
@@ -1325,10 +1351,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   constexpr int DPL = F::DPL;
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
   const int nw = a.sp_nw;
   const int r16 = lane & 15;
   const int kb = lane >> 4;
+  // (a scalar: the kv head, and with it every page address, stays in scalar
+  // registers)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // workgroup -> (its index within the sequence, sequence, unit); neighbouring
   // workgroups take different units
   const int unit = (int)blockIdx.x % a.units;
@@ -1381,7 +1409,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   c.Hkv = a.Hkv;
   c.hkv = hkv;
   c.seq_len = len;
-  const LaneOffsets<KVF, D, SB> lo = pt_lane_offsets<KVF, D, SB>(a, r16, kb);
+  LaneOffsets<KVF, D, SB> lo = pt_lane_offsets<KVF, D, SB>(a, r16, kb);
 
   float m_run = -INFINITY;  // per head r16 (replicated over kb)
   float l_run = 0.0f;
