@@ -114,7 +114,9 @@ int mk_q8_matvec_ws(const void* x, const uint8_t* w, const void* scales, const v
  * streams).  gate_out/up_out [M,N] (nullable) receive the two products;
  * mlp_out [M,N] (nullable) receives the fused SwiGLU epilogue
  * silu(gate)*up (ops/activation_ops.py:83-88) computed from the rounded
- * gate/up values.  At least one output must be non-NULL. */
+ * gate/up values.  At least one output must be non-NULL.  z_gate and z_up are
+ * nullable each by itself (NULL: no zero points); with one of the two alone
+ * the call takes the MFMA kernel of 16 rows a launch, or the generic one. */
 int mk_q4_gate_up(const void* x, const uint8_t* w_gate, const uint8_t* w_up,
                   const void* s_gate, const void* s_up, const void* z_gate, const void* z_up,
                   void* gate_out, void* up_out, void* mlp_out, int64_t M, int64_t N, int64_t K,
@@ -130,8 +132,9 @@ int mk_q8_gate_up(const void* x, const uint8_t* w_gate, const uint8_t* w_up,
  * add z = x + residual (z_out [M,K]), RMSNorm normed = z * rsqrt(mean(z^2) +
  * eps) * norm_w (normed_out [M,K]), then the gate/up products and SwiGLU as
  * mk_q4_gate_up / mk_q8_gate_up.  For q4 or q8 with an M = 1 fp16 row, K <=
- * 8192, fp16 norm weights and fp16 scales this is one launch (the norm runs inside
- * the gate/up kernel) and normed_out may be NULL; otherwise the norm kernel
+ * 8192, fp16 norm weights, fp16 scales and zero points for both matrices or
+ * neither this is one launch (the norm runs inside the gate/up kernel) and
+ * normed_out may be NULL; otherwise the norm kernel
  * and the gate/up kernel run in turn through normed_out, which is then
  * required (MK_ERR_INVALID when NULL).
  * norm_w_dtype: MK_DT_F16/BF16/F32. */

@@ -466,7 +466,7 @@ template <int BITS, int NMAT>
 bool gemm_rows_ok(const GemvArgs& a, int64_t M, int64_t gs) {
   bool ok = a.lg >= 5 && (int64_t)1 << a.lg == gs && (a.K % (128 / BITS)) == 0 && mk_aligned(a.x, 16) &&
             (int64_t)a.N * a.row_bytes < (1LL << 31) && (int64_t)a.N * a.G < (1LL << 30) &&
-            M * a.K < (1LL << 31);
+            M * a.K < (1LL << 31) && zeros_alike<NMAT>(a);
   for (int t = 0; t < NMAT; ++t) ok = ok && mk_aligned(a.w[t], 16);
   return ok;
 }

@@ -1136,7 +1136,7 @@ bool xk_eligible(const GemvArgs& a, int mt, int act_dt, int sc_dt) {
 template <int NMAT>
 bool tile_eligible(const GemvArgs& a, int act_dt, int sc_dt) {
   bool ok = act_dt == MK_DT_F16 && sc_dt == MK_DT_F16 && a.lg >= 5 && (a.K % 128) == 0 &&
-            mk_aligned(a.x, 16) && (size_t)a.row_bytes % 16 == 0;
+            mk_aligned(a.x, 16) && (size_t)a.row_bytes % 16 == 0 && zeros_alike<NMAT>(a);
   for (int t = 0; t < NMAT; ++t) ok = ok && mk_aligned(a.w[t], 16);
   return ok;
 }
@@ -1236,6 +1236,7 @@ bool dot_eligible(const GemvArgs& a, bool fast, int64_t mrows, int act_dt, int s
          (K % 32) == 0 && K <= 8 * 2048 && (a.G % 8) == 0 && (gpw % 8) == 0 &&
          (int64_t)NMAT * dot_rows<BITS, NMAT>() * 2 * (gpw / 8) <= 64 * DOT_SZ_VEC &&
          mk_aligned(a.s[0], 16) && mk_aligned(a.s[NMAT - 1], 16) &&
+         zeros_alike<NMAT>(a) &&
          (a.z[0] == nullptr || (mk_aligned(a.z[0], 16) && mk_aligned(a.z[NMAT - 1], 16)));
 }
 

@@ -196,7 +196,7 @@ struct GemvArgs {
   const void* x;         // [M, K]
   const uint8_t* w[2];   // [N, row_bytes]
   const void* s[2];      // [N, G]
-  const void* z[2];      // [N, G] or null
+  const void* z[2];      // [N, G] or null, each by itself
   const void* residual;  // [M, N] or null
   void* y0;              // EPI_NONE: y; EPI_RESIDUAL: y_mm (nullable); GATE_UP: gate (nullable)
   void* y1;              // EPI_RESIDUAL: out;  GATE_UP: up (nullable)
@@ -218,6 +218,14 @@ struct GemvArgs {
   float eps;
   RopeKV rk;             // EPI_ROPE_KV only
 };
+
+// Both matrices of a pair have zero points, or neither: what every kernel but
+// gemv_mfma_kernel and gemv_generic_kernel takes for granted (they test z[0]
+// and read both).
+template <int NMAT>
+inline bool zeros_alike(const GemvArgs& a) {
+  return NMAT == 1 || (a.z[0] == nullptr) == (a.z[1] == nullptr);
+}
 
 // --------------------------------------------------------------------------
 // shared epilogue: value(s) of output row n for activation row m

@@ -486,7 +486,8 @@ size_t few_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 template <int BITS, int NMAT>
 bool few_ok(const GemvArgs& a, int64_t M, int64_t gs, int sc_dt, size_t ws_bytes) {
   bool ok = sc_dt == MK_DT_F16 && a.lg >= 5 && (int64_t)1 << a.lg == gs && (a.K % 32) == 0 && M >= 1 &&
-            M <= (BITS == 4 ? 32 : 16) && a.N < (1 << 26) && a.K < (1 << 26) && mk_aligned(a.x, 16);
+            M <= (BITS == 4 ? 32 : 16) && a.N < (1 << 26) && a.K < (1 << 26) && mk_aligned(a.x, 16) &&
+            zeros_alike<NMAT>(a);
   for (int t = 0; t < NMAT; ++t) ok = ok && mk_aligned(a.w[t], 16);
   return ok && few_workspace_bytes(M, a.N, a.K) <= ws_bytes;
 }
