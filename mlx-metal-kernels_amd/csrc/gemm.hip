@@ -228,8 +228,9 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
       for (int j = 0; j < WC; ++j) lds_copy<16>(wsrc[j] + (k0 * BITS / 8 + 16 * wk16), wlds + slot + j * 1024);
     } else {
-      // the last, partial stage: chunks past K are zero, so that whatever
-      // codes they meet (the row's first, re-read) adds nothing
+      // the last, partial stage: chunks past K are zero, and the codes they
+      // meet (the row's first, re-read) are unpacked with a zero scale, so that
+      // they add nothing
 #pragma unroll
       for (int i = 0; i < XC; ++i) {
         uint8_t* const d = xd + i * 64 * WN * 16;
@@ -275,24 +276,40 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2)
     // SZ8: the group of this lane's 16 k (past K: the row's last one)
     const int grp = min(((st0 + it) * GK + 16 * kb) >> args.lg, G - 1);
     codes_t c[GNT];
+    ST sv[GNT], zv[GNT];
+#pragma unroll
+    for (int t = 0; t < GNT; ++t) {
+      c[t] = *reinterpret_cast<const codes_t*>(wb + wpos + t * 16 * CB);
+      zv[t] = (ST)0.0f;
+      if constexpr (SZ8) {
+        const uint8_t* const p = szlds + ((grp >> 3) & 1) * 2048 + (16 * t + r) * 16 + (grp & 7) * 2;
+        sv[t] = *reinterpret_cast<const ST*>(p);
+        if (has_z) zv[t] = *reinterpret_cast<const ST*>(p + 1024);
+      } else {
+        sv[t] = *reinterpret_cast<const ST*>(wb + spos + t * 64);
+        if (has_z) zv[t] = *reinterpret_cast<const ST*>(wb + spos + 256 + t * 64);
+      }
+    }
+    if ((st0 + it + 1) * GK > K) {
+      // The last, partial stage: lanes past K.  A weight that is none may be
+      // infinite once rounded, and infinity times the zero activation is NaN.
+      // (The asm keeps this a branch: as selects, every turn pays 2 % for it.)
+      const bool past = (st0 + it) * GK + 16 * kb >= K;
+      asm volatile("");
+#pragma unroll
+      for (int t = 0; t < GNT; ++t) {
+        sv[t] = past ? (ST)0.0f : sv[t];
+        zv[t] = past ? (ST)0.0f : zv[t];
+      }
+    }
     ExactGp<ST> ge[GNT];
     GpNat gp[GNT];
 #pragma unroll
     for (int t = 0; t < GNT; ++t) {
-      c[t] = *reinterpret_cast<const codes_t*>(wb + wpos + t * 16 * CB);
-      ST sv, zv = (ST)0.0f;
-      if constexpr (SZ8) {
-        const uint8_t* const p = szlds + ((grp >> 3) & 1) * 2048 + (16 * t + r) * 16 + (grp & 7) * 2;
-        sv = *reinterpret_cast<const ST*>(p);
-        if (has_z) zv = *reinterpret_cast<const ST*>(p + 1024);
-      } else {
-        sv = *reinterpret_cast<const ST*>(wb + spos + t * 64);
-        if (has_z) zv = *reinterpret_cast<const ST*>(wb + spos + 256 + t * 64);
-      }
       if constexpr (MAGIC) {
-        gp[t] = make_gp_nat<BITS>((f16)sv, (f16)zv);
+        gp[t] = make_gp_nat<BITS>((f16)sv[t], (f16)zv[t]);
       } else {
-        ge[t] = make_exact_gp<ST>(sv, zv);
+        ge[t] = make_exact_gp<ST>(sv[t], zv[t]);
       }
     }
     auto dequant = [&](int t, int h) {

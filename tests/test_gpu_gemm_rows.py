@@ -105,3 +105,28 @@ def test_product_unaligned_scales_and_saturation(dev, bits):
     assert torch.equal(fn(x, packed, off(s), off(z), group_size=g), want)
     big = fn(torch.full((40, K), 200.0, device=dev).half(), packed, s * 400, None, group_size=g)
     assert bool((big == 65504.0).all())
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("K,g", [(96, 32), (96, 64), (1056, 128), (2080, 32)])
+def test_product_past_k_with_large_weights(dev, bits, K, g):
+    """The last stage past K adds nothing, also where the last group's scale
+    would make an infinite fp16 weight of other codes than its own (they re-read
+    the row's first ones), and where the row's own first weights are infinite:
+    those give the saturated sum, as in the reference."""
+    gen = torch.Generator(device=dev).manual_seed(K + g)
+    M, N, top = 70, 70, 15 if bits == 4 else 255
+    codes = torch.full((N, K), top, dtype=torch.uint8, device=dev)
+    codes[:, (K - 1) // g * g:] = 2
+    s = torch.full((N, -(-K // g)), 1e-3, device=dev).half()
+    s[:, -1] = 2 * 65504.0 / top  # top * s is past fp16, the group's own 2 * s is not
+    packed = codes[:, 0::2] | (codes[:, 1::2] << 4) if bits == 4 else codes
+    x = (torch.randn((M, K), generator=gen, device=dev) * 0.01).half()
+    x[:, (K - 1) // g * g:] *= 0.01
+    fn = qo.q4_matvec_decode if bits == 4 else qo.q8_matvec_decode
+    _check(fn(x, packed.contiguous(), s, None, group_size=g), x, _rounded(codes, s, None, g, torch.float16),
+           torch.float16, (K, g))
+    s[:] = 1e-3
+    s[:, 0] = 2 * 65504.0 / top
+    got = fn(x.abs() + 1e-3, packed.contiguous(), s, None, group_size=g)
+    assert bool((got == 65504.0).all())
