@@ -209,6 +209,7 @@ __global__ __launch_bounds__(64 * FMAXW) __attribute__((amdgpu_waves_per_eu(XL ?
     gb[j] = kc >> args.lg;
   }
   const int g0 = k0 < K ? k0 >> args.lg : 0;  // LG > 0: K % FKW == 0, the wave's groups lie in the row
+  const bool idle = LG > 0 && k0 >= K;        // LG > 0: nor is a wave partly past K; its sums are zero (LG 0: see block)
   const bool has_z = args.z[0] != nullptr;
 
   u32x4 w[DU][FB][WV];
@@ -262,6 +263,13 @@ __global__ __launch_bounds__(64 * FMAXW) __attribute__((amdgpu_waves_per_eu(XL ?
     f16 sv, zv;
     sz_at<BITS, LG>(sz[u], j, kb, &sv, &zv);
     if (!has_z) zv = (f16)0.0f;
+    if constexpr (LG == 0) {
+      // blocks past K re-read real weights, which may be infinite once rounded:
+      // times the zero activations that would be NaN
+      const bool past = k0 + lane_k<BITS>(j, kb) >= K;
+      sv = past ? (f16)0.0f : sv;
+      zv = past ? (f16)0.0f : zv;
+    }
     GpMagic gp;
     ExactGp<f16> ge;
     if constexpr (MAGIC) {
@@ -306,7 +314,7 @@ __global__ __launch_bounds__(64 * FMAXW) __attribute__((amdgpu_waves_per_eu(XL ?
         }
       }
 #pragma unroll
-      for (int u = 0; u < DU; ++u) rb[(u * nw + wave) * 64 + lane] = acc[u];
+      for (int u = 0; u < DU; ++u) rb[(u * nw + wave) * 64 + lane] = idle ? (f32x4){0.f, 0.f, 0.f, 0.f} : acc[u];
     } else {
       // every buffer takes its next unit once it is used (unconditional loads:
       // the wait counts stay exact; past the run they re-read its last tile)
@@ -321,7 +329,8 @@ __global__ __launch_bounds__(64 * FMAXW) __attribute__((amdgpu_waves_per_eu(XL ?
         issue((t0 - t_begin) * NMAT + u + DU, u, u % NMAT);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) rb[((u * MT + mt) * nw + wave) * 64 + lane] = acc[mt];
+        for (int mt = 0; mt < MT; ++mt)
+          rb[((u * MT + mt) * nw + wave) * 64 + lane] = idle ? (f32x4){0.f, 0.f, 0.f, 0.f} : acc[mt];
       }
     }
     lds_barrier();

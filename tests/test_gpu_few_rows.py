@@ -77,3 +77,20 @@ def test_few_rows_unaligned_scales_and_no_workspace(dev, bits):
     _lib.launch(f"mk_q{bits}_matvec", dev, x.data_ptr(), packed.data_ptr(), s.data_ptr(), z.data_ptr(), None, None,
                 y.data_ptr(), M, N, K, g, _lib.DT_F16, _lib.DT_F16)
     _check(y, x, _rounded(codes, s, z, g, torch.float16), torch.float16, "no workspace")
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,K,g", [(6, 96, 32), (16, 544, 64), (8, 1056, 128), (16, 4608, 32), (7, 4608, 64), (5, 4608, 128)])
+def test_few_rows_infinite_weights_before_k_ends(dev, M, K, g, bits):
+    """Rows whose first weights are infinite in fp16 give the saturated sum, also
+    where blocks (or whole waves) past K re-read them against zero activations."""
+    N, top = 70, 15 if bits == 4 else 255
+    codes = torch.full((N, K), top, dtype=torch.uint8, device=dev)
+    s = torch.full((N, -(-K // g)), 1e-3, device=dev).half()
+    s[:, 0] = 2 * 65504.0 / top
+    packed = (codes[:, 0::2] | (codes[:, 1::2] << 4) if bits == 4 else codes).contiguous()
+    fn = qo.q4_matvec_decode if bits == 4 else qo.q8_matvec_decode
+    x = torch.full((M, K), 0.01, device=dev).half()
+    x[1::2] = -0.01
+    got = fn(x, packed, s, None, group_size=g)
+    assert bool((got[0::2] == 65504.0).all()) and bool((got[1::2] == -65504.0).all())
