@@ -5,6 +5,7 @@ from __future__ import annotations
 import os
 
 import torch
+from torch.autograd import forward_ad
 
 ACT_DTYPES = (torch.float16, torch.bfloat16)
 FLOAT_DTYPES = (torch.float16, torch.bfloat16, torch.float32, torch.float64)
@@ -39,6 +40,21 @@ def as_dense(t, dtype):
     if t is None or (t.dtype == dtype and t.is_contiguous()):
         return t
     return t.to(dtype).contiguous()
+
+
+def values_only(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel that reads the tensors' memory does all that tensor ops
+    would: no gradient to record, no forward-mode tangent, no function transform
+    (vmap, jvp, grad), no tracing, dispatch mode or tensor subclass."""
+    if (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None):  # (there even new tensors are wrapped)
+        return False
+    for t in tensors:
+        if type(t) not in (torch.Tensor, torch.nn.Parameter):
+            return False
+        if (t.requires_grad and torch.is_grad_enabled()) or forward_ad.unpack_dual(t).tangent is not None:
+            return False
+    return True
 
 
 def as_u8(t: torch.Tensor) -> torch.Tensor:

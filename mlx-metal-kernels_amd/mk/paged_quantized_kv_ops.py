@@ -26,6 +26,7 @@ from typing import Any
 import torch
 
 from . import _lib
+from ._common import values_only
 from .gqa_ops import _per_sequence_rope, _qkv_rope_update_prep, validate_gqa_heads
 from .kv_cache_ops import normalize_positions
 from .paged_kv_ops import _i32
@@ -237,11 +238,11 @@ def _hip_quantize_rows(pages: torch.Tensor, group_size: int, bits: int):
 def _hip_dequantize(codes: torch.Tensor, scales: torch.Tensor, group_size: int, bits: int, D: int):
     """mk_dequantize_kv of device codes [..., D | ceil(D/2)] with fp16 scales
     [..., ceil(D/group_size)] -> fp16 [..., D]; None for what the kernel does
-    not take (host tensors, other types or layouts, scales that need a
-    gradient), which stays with the tensor ops."""
+    not take (host tensors, other types or layouts, gradients, function
+    transforms and tracing), which stays with the tensor ops."""
     want = tuple(codes.shape[:-1])
     if (codes.device.type != "cuda" or scales.device != codes.device or codes.dtype != torch.uint8
-            or scales.dtype != torch.float16 or (scales.requires_grad and torch.is_grad_enabled()) or D <= 0
+            or scales.dtype != torch.float16 or not values_only(codes, scales) or D <= 0
             or group_size <= 0 or tuple(codes.shape) != want + (D if bits == 8 else (D + 1) // 2,)
             or tuple(scales.shape) != want + ((D + group_size - 1) // group_size,)):
         return None

@@ -66,3 +66,40 @@ def test_dequantize_leaves_other_forms_to_the_tensor_ops(dev):
     assert pq._hip_dequantize(codes.int(), scales, 64, 8, 64) is None
     assert pq._hip_dequantize(codes, scales, 32, 8, 64) is None  # two groups per row expected
     assert pq._hip_dequantize(codes[:0], scales[:0], 64, 8, 64).shape == (0, 64)
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+def test_dequantize_under_transforms(dev, bits):
+    """Forward-mode, jvp, vmap and reverse-mode of both dequantizers over the
+    scales: the tensor ops' values and tangents."""
+    import dataclasses
+
+    import torch.autograd.forward_ad as fwAD
+
+    import mk.quantized_kv_cache_ops as qc
+
+    gen = torch.Generator(device=dev).manual_seed(5)
+    x = torch.randn(3, 16, 2, 64, generator=gen, device=dev).half()
+    table = torch.arange(3, dtype=torch.int32, device=dev).reshape(1, 3)
+    paged = pq.quantize_kv_pages(x, x, table, torch.tensor([48], dtype=torch.int32, device=dev),
+                                 pq.PagedQuantizedKVConfig(bits=bits, page_size=16, group_size=32))
+    flat = qc.quantize_kv_cache(x, x, qc.QuantizedKVCacheConfig(bits=bits, group_size=32))
+    for cache, fn in ((paged, pq.dequantize_kv_pages), (flat, qc.dequantize_kv_cache)):
+        f = lambda s: fn(dataclasses.replace(cache, k_scales=s))[0]
+        s, t = cache.k_scales, torch.randn(cache.k_scales.shape, generator=gen, device=dev).half()
+        off = fn(dataclasses.replace(cache, k_scales=torch.ones_like(s)))[0].float()  # code - 128 | 8
+        want_t = (off * t.float().repeat_interleave(32, dim=-1)).half()  # scales are positive
+        with fwAD.dual_level():
+            out = fwAD.unpack_dual(f(fwAD.make_dual(s, t)))
+            assert torch.equal(out.primal, f(s)) and torch.equal(out.tangent, want_t)
+        val, tan = torch.func.jvp(f, (s,), (t,))
+        assert torch.equal(val, f(s)) and torch.equal(tan, want_t)
+        sg = s.clone().requires_grad_(True)
+        f(sg).float().sum().backward()
+        want_g = off.half().float().unflatten(-1, (-1, 32)).sum(-1)
+        assert torch.allclose(sg.grad.float(), want_g, rtol=2e-3, atol=1e-2)
+    rows = torch.stack([paged.k_scales, paged.k_scales * 2])
+    got = torch.func.vmap(lambda s: pq.dequantize_kv_pages(
+        dataclasses.replace(paged, k_scales=s, v_scales=s))[0])(rows)
+    for i in range(2):
+        assert torch.equal(got[i], pq.dequantize_kv_pages(dataclasses.replace(paged, k_scales=rows[i]))[0])
