@@ -26,7 +26,7 @@ from typing import Any
 import torch
 
 from . import _lib
-from ._common import values_only
+from ._common import ci_safe_mode_enabled, values_only
 from .gqa_ops import _per_sequence_rope, _qkv_rope_update_prep, validate_gqa_heads
 from .kv_cache_ops import normalize_positions
 from .paged_kv_ops import _i32
@@ -265,6 +265,12 @@ def _unpacked_codes(paged_qkv: PagedQuantizedKVCache, which: str, D: int) -> tor
 
 def dequantize_kv_pages(paged_qkv: PagedQuantizedKVCache):
     """ops/paged_quantized_kv_ops.py:295-341 -> fp16 (K, V)."""
+    return _dequantize_pages(paged_qkv, not ci_safe_mode_enabled())
+
+
+def _dequantize_pages(paged_qkv: PagedQuantizedKVCache, kernel: bool):
+    """``kernel`` False: by tensor ops alone, for the reference backends, which
+    must not depend on the kernels they are compared with."""
     paged_qkv = paged_qkv.validate()
     orig = paged_qkv.original_page_shape
     if orig is None:
@@ -272,7 +278,7 @@ def dequantize_kv_pages(paged_qkv: PagedQuantizedKVCache):
     D = orig[3]
 
     def values(which, codes, scales):
-        out = _hip_dequantize(codes, scales, paged_qkv.group_size, paged_qkv.bits, D)
+        out = _hip_dequantize(codes, scales, paged_qkv.group_size, paged_qkv.bits, D) if kernel else None
         if out is None:
             out = _dequant_last_dim(_unpacked_codes(paged_qkv, which, D), scales, paged_qkv.group_size,
                                     paged_qkv.bits, D).to(torch.float16)
@@ -383,7 +389,7 @@ def reference_paged_quantized_kv_gqa_decode_attention(q, paged_qkv: PagedQuantiz
     lengths_arr, B, MAX_S, PAGE_SIZE, MAX_BLOCKS, Hq, Hkv, D = _validate_paged_quantized_decode_inputs(q, paged_qkv)
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    K_deq, V_deq = dequantize_kv_pages(paged_qkv)
+    K_deq, V_deq = _dequantize_pages(paged_qkv, False)
     bt = paged_qkv.block_table.to(K_deq.device)
     Kc, valid = _gather_pages(K_deq, bt, MAX_S)
     Vc, _ = _gather_pages(V_deq, bt, MAX_S)

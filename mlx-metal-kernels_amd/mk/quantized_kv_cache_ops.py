@@ -25,6 +25,7 @@ from typing import Any
 import torch
 
 from . import _contig, _lib
+from ._common import ci_safe_mode_enabled
 from .gqa_ops import validate_gqa_heads
 from .kv_cache_ops import normalize_positions
 from .paged_kv_ops import _masked_attention
@@ -168,12 +169,17 @@ def _codes(cache: QuantizedKVCache, which: str, D: int) -> torch.Tensor:
 def dequantize_kv_cache(qkv_cache: QuantizedKVCache):
     """ops/quantized_kv_cache_ops.py:280-313: (code - 128|8) * |s| in fp32,
     rounded to fp16, for every position."""
+    return _dequantize_cache(qkv_cache, not ci_safe_mode_enabled())
+
+
+def _dequantize_cache(qkv_cache: QuantizedKVCache, kernel: bool):
+    """``kernel`` False: by tensor ops alone, for the reference backend."""
     qkv_cache = qkv_cache.validate()
     B, S, H, D = _geometry(qkv_cache)
     g, bits = qkv_cache.group_size, qkv_cache.bits
 
     def values(which, codes, scales):
-        out = _hip_dequantize(codes, scales, g, bits, D)
+        out = _hip_dequantize(codes, scales, g, bits, D) if kernel else None
         return _dequant_last_dim(_codes(qkv_cache, which, D), scales, g, bits, D).to(torch.float16) if out is None else out
 
     K = values("k", qkv_cache.k_q, qkv_cache.k_scales)
@@ -222,7 +228,7 @@ def reference_quantized_kv_gqa_decode_attention(q, qkv_cache: QuantizedKVCache, 
     lengths_arr, B, MAX_S, Hq, Hkv, D = _validate_quantized_decode_inputs(q, qkv_cache, lengths)
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    K_deq, V_deq = dequantize_kv_cache(qkv_cache)
+    K_deq, V_deq = _dequantize_cache(qkv_cache, False)
     valid = torch.ones((B, MAX_S), dtype=torch.bool, device=q.device)
     out = _masked_attention(q[:, 0], K_deq.to(q.device), V_deq.to(q.device), lengths_arr, valid, scale)
     return out.unsqueeze(1).to(q.dtype)

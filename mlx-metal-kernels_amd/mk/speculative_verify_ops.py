@@ -35,7 +35,7 @@ from .llama_stack_ops import (LlamaStackCache, LlamaStackWeights, embed_token_id
                               llama_stack_decode_step)
 from . import _contig
 from .paged_kv_ops import _i32
-from .paged_quantized_kv_ops import PagedQuantizedKVCache, _check_kernel_layout, dequantize_kv_pages
+from .paged_quantized_kv_ops import PagedQuantizedKVCache, _check_kernel_layout, _dequantize_pages
 
 _ACT = (torch.float16, torch.bfloat16)
 
@@ -271,7 +271,7 @@ def paged_quantized_verify_attention(q, paged_qkv: PagedQuantizedKVCache, length
     B, W, ln = _verify_shapes(q, paged_qkv.block_table, src, max_s)
     sc = 1.0 / math.sqrt(q.shape[3]) if scale is None else scale
     if backend.lower() == "reference":
-        Kp, Vp = dequantize_kv_pages(paged_qkv)
+        Kp, Vp = _dequantize_pages(paged_qkv, False)
         return reference_paged_verify_attention(q, Kp.to(q.dtype), Vp.to(q.dtype), paged_qkv.block_table, ln, sc)
     if backend.lower() not in ("auto", "metal"):
         raise ValueError("backend must be one of 'reference', 'metal', 'auto'")
