@@ -121,11 +121,14 @@ constexpr size_t gemm_lds_bytes(int bits, int mt, int wn, int wk, bool sz8, int 
 // 0) are copied 8 groups at a time.  Otherwise each stage copies every row's
 // two (a group of 32 spans half a stage) by themselves: 64 separate lines per
 // copy instruction where the codes touch 32 and the activations 8.
-template <int BITS, typename AT, typename ST, int NMAT, int EPI, bool SZ8, int MT, int WN, int WK, int RING>
+//
+// MAGIC: fp16 weights by the exponent trick, which holds a fractional zero
+// point's part in fp16; otherwise (q - z) * s in fp32, rounded once.
+template <int BITS, typename AT, typename ST, int NMAT, int EPI, bool SZ8, bool MAGIC, int MT, int WN, int WK, int RING>
 __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2))) void gemm_rows_kernel(
     const GemvArgs args) {
   static_assert(!SZ8 || sizeof(ST) == 2, "SZ8 copies 8 fp16 values");
-  constexpr bool MAGIC = sizeof(ST) == 2 && __is_same(AT, f16);
+  static_assert(!MAGIC || (sizeof(ST) == 2 && __is_same(AT, f16)), "MAGIC unpacks to fp16 with fp16 scales");
   constexpr int XC = MT * 16 * (GK / 8) / (64 * WN);    // 16-byte activation chunks copied per thread and stage
   constexpr int WC = gemm_code_bytes(BITS) / (64 * 16); // 16-byte code copies per thread and stage
   constexpr int COPIES = XC + WC + (SZ8 ? 0 : 4);       // copies per wave and stage (SZ8: 2 more now and then)
@@ -430,7 +433,7 @@ inline int gemm_plan(int bits, int M, int N, int K, int nmat, int cus, float* us
   return best;
 }
 
-template <int BITS, typename AT, typename ST, int NMAT, int EPI, bool SZ8, int MT, int WN, int WK, int RING>
+template <int BITS, typename AT, typename ST, int NMAT, int EPI, bool SZ8, bool MAGIC, int MT, int WN, int WK, int RING>
 int launch_plan(GemvArgs a, hipStream_t st) {
   const int rows = WN * 16 * GNT / NMAT;
   a.rg = (a.M + 16 * MT - 1) / (16 * MT);
@@ -439,16 +442,16 @@ int launch_plan(GemvArgs a, hipStream_t st) {
   if (grid >= (1LL << 31)) return MK_ERR_UNSUPPORTED;
   constexpr size_t lds = gemm_lds_bytes(BITS, MT, WN, WK, SZ8, RING);
   static_assert(lds <= 160 * 1024, "the ring fits a CU's LDS");
-  gemm_rows_kernel<BITS, AT, ST, NMAT, EPI, SZ8, MT, WN, WK, RING>
+  gemm_rows_kernel<BITS, AT, ST, NMAT, EPI, SZ8, MAGIC, MT, WN, WK, RING>
       <<<dim3((unsigned)grid), dim3(64 * WN * WK), lds, st>>>(a);
   MK_CHECK_LAUNCH();
   return MK_OK;
 }
 
-template <int BITS, typename AT, typename ST, int NMAT, int EPI, bool SZ8>
+template <int BITS, typename AT, typename ST, int NMAT, int EPI, bool SZ8, bool MAGIC>
 int launch_types(const GemvArgs& a, hipStream_t st) {
-#define MK_PLAN(I, RING4, RING8)                                                                            \
-  return launch_plan<BITS, AT, ST, NMAT, EPI, SZ8, kGemmShapes[I].mt, kGemmShapes[I].wn, kGemmShapes[I].wk, \
+#define MK_PLAN(I, RING4, RING8)                                                                      \
+  return launch_plan<BITS, AT, ST, NMAT, EPI, SZ8, MAGIC, kGemmShapes[I].mt, kGemmShapes[I].wn, kGemmShapes[I].wk, \
                      BITS == 4 ? RING4 : RING8>(a, st)
   // ring depths: as many stages as fit
   switch (gemm_plan(BITS, a.M, a.N, a.K, NMAT, device_cu_count())) {
@@ -464,13 +467,25 @@ int launch_types(const GemvArgs& a, hipStream_t st) {
 
 template <int BITS, typename AT, typename ST, int NMAT, int EPI>
 int launch_scales(const GemvArgs& a, hipStream_t st) {
+  // fp16 weights by the exponent trick where gemv_mfma_kernel would take it too;
+  // exact for the layouts that were gemv_generic_kernel's alone, so that no
+  // weight is held in fewer bits than there.  (Exact everywhere: 2 x 14336 x 4096
+  // at 64 rows 35.4 -> 36.4 us, q8 4096 x 14336 at 300 rows 97 -> 105.)
+  constexpr bool F16 = sizeof(ST) == 2 && __is_same(AT, f16);
+  const bool exact = a.K % QFmt<BITS>::KL != 0;
   if constexpr (sizeof(ST) == 2) {
     bool sz8 = (a.G % 8) == 0;
     for (int t = 0; t < NMAT; ++t)
       sz8 = sz8 && mk_aligned(a.s[t], 16) && (a.z[0] == nullptr || mk_aligned(a.z[t], 16));
-    if (sz8) return launch_types<BITS, AT, ST, NMAT, EPI, true>(a, st);
+    if (sz8) {
+      if constexpr (F16)
+        if (exact) return launch_types<BITS, AT, ST, NMAT, EPI, true, false>(a, st);
+      return launch_types<BITS, AT, ST, NMAT, EPI, true, F16>(a, st);
+    }
   }
-  return launch_types<BITS, AT, ST, NMAT, EPI, false>(a, st);
+  if constexpr (F16)
+    if (exact) return launch_types<BITS, AT, ST, NMAT, EPI, false, false>(a, st);
+  return launch_types<BITS, AT, ST, NMAT, EPI, false, F16>(a, st);
 }
 
 }  // namespace

@@ -411,7 +411,11 @@ __device__ __forceinline__ u32x4 dq_exact8(uint32_t u0, uint32_t u1, const Exact
   }
   u32x4 r;
 #pragma unroll
-  for (int p = 0; p < 4; ++p) r[p] = pack2<AT>(c[2 * p], c[2 * p + 1]);
+  for (int p = 0; p < 4; ++p) {
+    // (as a vector: v_fma_mixlo and v_fma_mixhi write the pair, 13 instructions)
+    if constexpr (__is_same(AT, f16)) r[p] = bitcast<uint32_t>((f16x2){(f16)c[2 * p], (f16)c[2 * p + 1]});
+    else r[p] = pack2<AT>(c[2 * p], c[2 * p + 1]);
+  }
   return r;
 }
 

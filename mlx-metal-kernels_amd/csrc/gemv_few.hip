@@ -139,13 +139,15 @@ struct FewArgs {
 
 // XL: one tile per workgroup, activations read from LDS as they are used (at
 // most XL rows of them), so that two workgroups of 128 registers share a CU
-template <int BITS, typename AT, int NMAT, int MT, int DU, int LG, int EPI, int XL>
+// MAGIC: fp16 weights by the exponent trick, which holds a fractional zero
+// point's part in fp16; otherwise (q - z) * s in fp32, rounded once
+template <int BITS, typename AT, int NMAT, int MT, int DU, int LG, bool MAGIC, int EPI, int XL>
 __global__ __launch_bounds__(64 * FMAXW) __attribute__((amdgpu_waves_per_eu(XL ? 4 : 2))) void gemv_few_kernel(
     const FewArgs fa) {
   static_assert(DU % NMAT == 0, "a ring turn holds whole tiles");
   static_assert(!XL || (MT == 1 && DU == NMAT), "XL: one tile");
   constexpr int XROWS = XL ? XL : 16;
-  constexpr bool MAGIC = __is_same(AT, f16);
+  static_assert(!MAGIC || __is_same(AT, f16), "MAGIC unpacks to fp16");
   constexpr int WV = BITS == 4 ? 1 : 2;  // 16-byte code vectors per lane and block
   constexpr int RT = DU / NMAT;          // tiles per ring turn
   const GemvArgs& args = fa.g;
@@ -410,7 +412,7 @@ inline FewPlan few_plan(int N, int K, int cus) {
   return p;
 }
 
-template <int BITS, typename AT, int NMAT, int MT, int DU, int LG, int EPI, int XL>
+template <int BITS, typename AT, int NMAT, int MT, int DU, int LG, bool MAGIC, int EPI, int XL>
 int few_launch(const GemvArgs& a, float* ws, hipStream_t st) {
   FewPlan p = few_plan(a.N, a.K, device_cu_count());
   if (XL) p.runs = p.tiles;
@@ -421,7 +423,7 @@ int few_launch(const GemvArgs& a, float* ws, hipStream_t st) {
   f.nw = p.nw;
   f.runs = p.runs;
   f.tiles = p.tiles;
-  gemv_few_kernel<BITS, AT, NMAT, MT, DU, LG, EPI, XL>
+  gemv_few_kernel<BITS, AT, NMAT, MT, DU, LG, MAGIC, EPI, XL>
       <<<dim3((unsigned)(p.runs * p.slices)), dim3(64 * p.nw), few_lds_bytes(p.nw, MT, DU, XL), st>>>(f);
   MK_CHECK_LAUNCH();
   if (p.slices > 1) {
@@ -432,7 +434,7 @@ int few_launch(const GemvArgs& a, float* ws, hipStream_t st) {
   return MK_OK;
 }
 
-template <int BITS, typename AT, int NMAT, int EPI, int LG>
+template <int BITS, typename AT, int NMAT, int EPI, int LG, bool MAGIC = __is_same(AT, f16)>
 int few_columns(const GemvArgs& a, float* ws, hipStream_t st) {
   const FewPlan p = few_plan(a.N, a.K, device_cu_count());
   const int run = (p.tiles + p.runs - 1) / p.runs;  // tiles of the longest run
@@ -445,31 +447,37 @@ int few_columns(const GemvArgs& a, float* ws, hipStream_t st) {
   constexpr bool ONE = NMAT == 2 ? BITS == 4 && !__is_same(AT, f16) : BITS == 8 || !__is_same(AT, f16);
   if constexpr (ONE) {
     if (a.M <= 8 && (int64_t)p.tiles * p.slices <= 4 * device_cu_count()) {
-      if (a.M <= 4) return few_launch<BITS, AT, NMAT, 1, NMAT, LG, EPI, 4>(a, ws, st);
-      return few_launch<BITS, AT, NMAT, 1, NMAT, LG, EPI, 8>(a, ws, st);
+      if (a.M <= 4) return few_launch<BITS, AT, NMAT, 1, NMAT, LG, MAGIC, EPI, 4>(a, ws, st);
+      return few_launch<BITS, AT, NMAT, 1, NMAT, LG, MAGIC, EPI, 8>(a, ws, st);
     }
   }
   // the ring: no deeper than the run is long, and what the registers hold
   // beside the activations
   if (a.M <= 16) {
     if constexpr (BITS == 4) {
-      if (run * NMAT > 2) return few_launch<BITS, AT, NMAT, 1, 4, LG, EPI, 0>(a, ws, st);
+      if (run * NMAT > 2) return few_launch<BITS, AT, NMAT, 1, 4, LG, MAGIC, EPI, 0>(a, ws, st);
     }
-    if (NMAT == 2 || run > 1) return few_launch<BITS, AT, NMAT, 1, 2, LG, EPI, 0>(a, ws, st);
-    if constexpr (NMAT == 1) return few_launch<BITS, AT, NMAT, 1, 1, LG, EPI, 0>(a, ws, st);
+    if (NMAT == 2 || run > 1) return few_launch<BITS, AT, NMAT, 1, 2, LG, MAGIC, EPI, 0>(a, ws, st);
+    if constexpr (NMAT == 1) return few_launch<BITS, AT, NMAT, 1, 1, LG, MAGIC, EPI, 0>(a, ws, st);
   }
   if constexpr (BITS == 4) {
     if constexpr (NMAT == 1) {
-      if (run > 2) return few_launch<BITS, AT, NMAT, 2, 3, LG, EPI, 0>(a, ws, st);
-      if (run == 1) return few_launch<BITS, AT, NMAT, 2, 1, LG, EPI, 0>(a, ws, st);
+      if (run > 2) return few_launch<BITS, AT, NMAT, 2, 3, LG, MAGIC, EPI, 0>(a, ws, st);
+      if (run == 1) return few_launch<BITS, AT, NMAT, 2, 1, LG, MAGIC, EPI, 0>(a, ws, st);
     }
-    return few_launch<BITS, AT, NMAT, 2, 2, LG, EPI, 0>(a, ws, st);
+    return few_launch<BITS, AT, NMAT, 2, 2, LG, MAGIC, EPI, 0>(a, ws, st);
   }
   return MK_ERR_UNSUPPORTED;
 }
 
 template <int BITS, typename AT, int NMAT, int EPI>
 int few_groups(const GemvArgs& a, float* ws, hipStream_t st) {
+  if constexpr (BITS == 4 && __is_same(AT, f16) && EPI != EPI_ROPE_KV) {
+    // the layouts that were gemv_generic_kernel's alone: no weight in fewer bits
+    // than there (2 x 14336 x 4064 at 32 rows 30.1 us, 28.4 by the exponent trick;
+    // exact everywhere would cost 21.0 -> 23.4 at 8 rows of 2 x 14336 x 4096)
+    if (a.K % QFmt<BITS>::KL) return few_columns<BITS, AT, NMAT, EPI, 0, false>(a, ws, st);
+  }
   bool v16 = (a.G % 8) == 0 && (a.K % FKW) == 0, v8 = (a.G % 4) == 0 && (a.K % FKW) == 0;
   for (int t = 0; t < NMAT; ++t) {
     v16 = v16 && mk_aligned(a.s[t], 16) && mk_aligned(a.z[t], 16);
