@@ -98,7 +98,7 @@ int mk_q8_matvec(const void* x, const uint8_t* w, const void* scales, const void
                  int64_t group_size, int act_dtype, int scale_dtype, void* stream);
 
 /* The same with a workspace (16-byte aligned, any content) of
- * mk_matvec_workspace_bytes(M, N, K) bytes: 0 unless M <= 64 and K > 4096,
+ * mk_matvec_workspace_bytes(M, N, K) bytes: 0 unless M <= 68 and K > 4096,
  * where it lets passes of up to 32 rows split K over workgroups (the fp32 sums of the
  * slices go through it).  Without one such calls take the kernels that walk
  * whole rows. */

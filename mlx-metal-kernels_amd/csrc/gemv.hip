@@ -1250,9 +1250,19 @@ inline int dot_waves(int64_t K) {
 // up to 32 rows through the kernels here)
 constexpr int64_t kGemmMinRows = 33;
 
+// Rows of a whole pass: the 1-4 rows (q8: 2) that a batch leaves past its last
+// one take the v_dot2 kernel, which does not round W, as when every batch ran in
+// passes.  (16 where two column tiles' partial sums and a pair's 128 groups of
+// 32 did not fit LDS together.)
+template <int BITS, int NMAT>
+inline int64_t pass_rows(int64_t N, int64_t K, int64_t gs) {
+  const bool pair32 = BITS == 4 && NMAT == 2 && K == 4096 && gs == 32 && N % 16 == 0 && N >= 4096;
+  return K % 128 != 0 || pair32 ? 16 : 32;
+}
+
 template <int BITS, int NMAT, int EPI>
 int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int act_dt, int sc_dt,
-                  hipStream_t st, float* ws = nullptr, size_t ws_bytes = 0) {
+                  hipStream_t st, float* ws = nullptr, size_t ws_bytes = 0, int64_t product_rows = kGemmMinRows) {
   using F = QFmt<BITS>;
   MK_REQUIRE(M >= 0 && N > 0 && K > 0 && gs > 0);
   MK_REQUIRE(act_dt == MK_DT_F16 || act_dt == MK_DT_BF16);
@@ -1286,6 +1296,21 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
     // fp16 projections on the fast layouts only (the caller falls back)
     if (act_dt != MK_DT_F16 || sc_dt != MK_DT_F16 || !fast) return MK_ERR_UNSUPPORTED;
   }
+  {
+    const int64_t pass = pass_rows<BITS, NMAT>(N, K, gs), tail = M % pass;
+    if (M > pass && dot_eligible<BITS, NMAT>(a, fast, tail, act_dt, sc_dt)) {
+      // us at 33 / 36 / 65 rows, all rows in one form -> this, q4 g64:
+      // 2 x 14336 x 4096 36 / 35 / 53 -> 35 / 42 / 47, 6144 x 4096 18 / 18 / 22
+      // -> 16 / 18 / 26, 4096 x 14336 35 / 36 / 67 -> 28 / 32 / 48
+      rc = gemv_dispatch<BITS, NMAT, EPI>(a, M - tail, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes, BITS == 4 ? 32 : 33);
+      if (rc != MK_OK) return rc;
+      GemvArgs b = a;
+      b.M = (int)tail;
+      rows_from(b, M - tail);
+      b.kw = dot_waves(K);
+      return launch_dot<BITS, NMAT, EPI>(b, st);
+    }
+  }
   // The few-row kernel takes up to 32 rows a pass (8-bit codes: 16) of what
   // the v_dot2 kernel does not.  From kGemmMinRows rows one product of all
   // rows, unless two passes take less: few output rows over a long K leave the
@@ -1301,8 +1326,10 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
                      few_ok<BITS, NMAT>(a, M < kPass ? M : kPass, gs, sc_dt, ws_bytes);
     const bool wide8 = BITS == 8 && M > kPass;
     if constexpr (EPI != EPI_ROPE_KV) {
-      bool product = (M >= kGemmMinRows || (wide8 && NMAT == 2)) && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
-      if (product && few && M >= kGemmMinRows && BITS == 4 && NMAT == 1) {
+      bool product = (M >= product_rows || (wide8 && NMAT == 2)) && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
+      if (product && few && M <= kPass) {
+        product = false;  // one pass
+      } else if (product && few && M >= kGemmMinRows && BITS == 4 && NMAT == 1) {
         const float pass = act_dt == MK_DT_F16 ? 4.5f + 3.0e-7f * (float)N * (float)K : 4.0f + 4.3e-7f * (float)N * (float)K;
         product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 2.0f * pass;
       }

@@ -494,7 +494,7 @@ int few_groups(const GemvArgs& a, float* ws, hipStream_t st) {
 namespace mkq {
 
 size_t few_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M > 32 && M <= 64) M = 32;  // two passes
+  if (M > 32 && M <= 68) M = 32;  // two passes (and up to 4 rows past them)
   if (M < 1 || M > 32 || N < 1 || K < 1 || N >= (1LL << 26) || K >= (1LL << 26)) return 0;
   const FewPlan p = few_plan((int)N, (int)K, device_cu_count());
   return p.slices > 1 ? (size_t)p.slices * M * N * sizeof(float) : 0;

@@ -213,7 +213,7 @@ def _hip_mlp_block(x, residual, norm_weight, gate_w, up_w, down_w, gate_scales, 
     # the down projection's workspace, then z and normed [rows, D] and the
     # hidden activations [rows, I], each from a 256-byte boundary
     ws_b = 0
-    if rows <= 64 and out_dim > 4096:
+    if rows <= 68 and out_dim > 4096:
         ws_b = (_lib.load().mk_matvec_workspace_bytes(rows, k_dim, out_dim) + 255) & -256
     row_b = (2 * rows * k_dim + 255) & -256
     scratch = torch.empty(ws_b + 2 * row_b + 2 * rows * out_dim, dtype=torch.uint8, device=dev)

@@ -275,7 +275,7 @@ def _hip_matvec(bits, x2d, w, scales, zeros, group_size, residual=None, want_mm=
     # fp32 sums of K slices (few rows of a long K); from the allocator, so it
     # lives and is reused in this stream's order
     ws, ws_bytes = None, 0
-    if M <= 64 and K > 4096:
+    if M <= 68 and K > 4096:
         ws_bytes = int(_lib.load().mk_matvec_workspace_bytes(M, N, K))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
     if residual is None:

@@ -9,7 +9,7 @@ import torch
 
 import mk.quant_ops as qo
 from mk import _lib
-from tests.test_gpu_gemm_rows import _check, _rounded, _weight
+from tests.test_gpu_gemm_rows import _check, _check_rows, _rounded, _weight
 
 pytestmark = pytest.mark.gpu
 
@@ -29,9 +29,8 @@ def test_few_rows(dev, M, N, K, bits, dtype):
     fn = qo.q4_matvec_decode if bits == 4 else qo.q8_matvec_decode
     for g, zeros in ((64, "whole"), (32, "whole"), (128, "none"), (256, "whole")):
         codes, packed, s, z = _weight(gen, dev, N, K, bits, g, torch.float16, zeros)
-        W = _rounded(codes, s, z, g, dtype)
         got = fn(x, packed, s, z, group_size=g)
-        _check(got, x, W, dtype, f"M{M} N{N} K{K} q{bits} g{g} {zeros}")
+        _check_rows(got, x, codes, s, z, g, bits, f"M{M} N{N} K{K} q{bits} g{g} {zeros}")
         res = torch.randn((M, N), generator=gen, device=dev).to(dtype)
         mm, out = qo.q_matvec_residual(x, packed, s, z, res, bits=bits, group_size=g, want_mm=True)
         assert torch.equal(mm, got)
