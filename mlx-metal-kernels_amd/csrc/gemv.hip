@@ -1314,11 +1314,12 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
   // The few-row kernel takes up to 32 rows a pass (8-bit codes: 16) of what
   // the v_dot2 kernel does not.  From kGemmMinRows rows one product of all
   // rows, unless two passes take less: few output rows over a long K leave the
-  // product 64 workgroups (4096 x 14336 at 40 rows 66 us against 44; a pass of
-  // 17-32 rows takes 4.5 us + 0.30 ns per 1000 weights for q4 fp16, 4 + 0.43
-  // for bf16).  17-32 rows over 8-bit codes: the product for gate/up (two
-  // passes 70 us, the tile kernel 65), two passes for bf16 (47 against 65 at
-  // 4096 x 14336), the tile kernel below for fp16.
+  // product 64 workgroups (4096 x 14336 at 40 rows 66 us against 34; a pass of
+  // 17-32 rows takes 6.5 us + 0.14 ns per 1000 weights for q4 fp16, 6.3 + 0.175
+  // for bf16, and 3.3 for the sum of K slices).  17-32 rows over 8-bit codes: the
+  // product for gate/up (2 x 14336 x 4096 40 us, two passes 66, the tile kernel
+  // 65), two passes for bf16 (44 against 65 at 4096 x 14336), the tile kernel
+  // below for fp16.
   {
     constexpr int64_t kPass = BITS == 4 ? 32 : 16;
     const bool few = M <= 2 * kPass && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
@@ -1330,7 +1331,8 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
       if (product && few && M <= kPass) {
         product = false;  // one pass
       } else if (product && few && M >= kGemmMinRows && BITS == 4 && NMAT == 1) {
-        const float pass = act_dt == MK_DT_F16 ? 4.5f + 3.0e-7f * (float)N * (float)K : 4.0f + 4.3e-7f * (float)N * (float)K;
+        const float weights = (float)N * (float)K, sum = K > 4096 ? 3.3f : 0.0f;
+        const float pass = act_dt == MK_DT_F16 ? 6.5f + 1.4e-7f * weights + sum : 6.3f + 1.75e-7f * weights + sum;
         product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 2.0f * pass;
       }
       if (product) {

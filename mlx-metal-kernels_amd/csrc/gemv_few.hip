@@ -8,7 +8,7 @@
 // run of 16-row weight tiles.  Per tile and matrix (a "unit") a lane loads 16
 // bytes of codes for each 128 k (32 k of row r; 32 bytes for 8 bits) and the
 // groups of its row and k, and the units run in a ring of DU register buffers
-// -- 100 to 200 KB in flight per CU -- without a barrier: the waves meet once
+// -- 40 KB in flight per CU and unit -- without a barrier: the waves meet once
 // per ring turn, when their partial tiles are added through LDS.
 // Longer rows are cut into K slices of at most 4096 k whose fp32 sums go to a
 // workspace, added (with the residual) by a second kernel.
@@ -17,13 +17,14 @@
 // there to the operand layout; read straight into it, every load instruction
 // touches 64 separate 64-byte pieces.
 //
-// Measured, us, the kernels before -> this (gate/up + SwiGLU 2 x 14336 x 4096 |
-// 4096 x 14336 + residual | 6144 x 4096 | 4096 x 4096, g64, q8 g32):
-//   q4 fp16  8 rows  22.7 -> 20.6 | 18.4 -> 16.7 | 10.8 -> 8.6 | 8.0 -> 6.4
-//   q4 fp16 32 rows  30.1 -> 23.6 | 35.3 -> 22.2 | 16.9 -> 12.2 | 13.7 -> 9.8
-//   q4 bf16  4 rows  36.1 -> 26.1 | 21.2 -> 17.2 | 12.7 ->  9.2 | 9.1 -> 6.0
-//   q4 bf16 32 rows  78.8 -> 29.7 | 52.9 -> 25.1 | 32.2 -> 12.2 | 19.7 -> 9.0
-//   q8 fp16  8 rows  46.4 -> 34.3 | 28.3 -> 20.6 | 16.3 -> 11.2 | 10.2 -> 8.3
+// Measured, us in a graph over weights that no cache holds, the kernels before
+// -> this (gate/up + SwiGLU 2 x 14336 x 4096 | 4096 x 14336 | 6144 x 4096 | 4096 x
+// 4096, g64):
+//   q4 fp16  8 rows  19.3 -> 19.7 | 16.2 -> 14.9 |  9.1 ->  8.2 |  7.0 -> 5.5
+//   q4 fp16 32 rows  26.6 -> 23.4 | 33.2 -> 17.9 | 14.8 -> 11.1 | 12.7 -> 8.5
+//   q4 bf16  4 rows  34.9 -> 24.7 | 20.0 -> 17.5 | 11.9 ->  9.2 |  8.1 -> 6.6
+//   q4 bf16 32 rows  77.9 -> 28.9 | 50.1 -> 20.4 | 30.4 -> 12.3 | 18.2 -> 8.6
+//   q8 fp16  8 rows  46.0 -> 31.9 | 26.6 -> 22.1 | 15.6 -> 11.2 |  9.3 -> 8.4
 // What is left is the stream: 128256 x 4096 at 8 rows takes 68 us (78 before),
 // 60 without the unpacking and products, 65 without the turns' barriers.
 #include "common.h"
@@ -440,31 +441,34 @@ int few_columns(const GemvArgs& a, float* ws, hipStream_t st) {
   const int run = (p.tiles + p.runs - 1) / p.runs;  // tiles of the longest run
   // Up to 8 rows of the forms whose unpacking weighs most, while tiles are
   // few: one tile per workgroup (XL), two workgroups a CU.  Against the ring,
-  // us: bf16 q4 MLP block of 4096 and 14336 44.4 / 47.9 at 4 rows, 47.3 / 48.7
-  // at 8, 4096 x 14336 17.0 / 18.8 at 4; at 8 rows q8 g32 fp16 6144 x 4096 11.2 / 14.1, 4096 x 4096 8.3 / 9.3.  The ring
-  // is ahead for fp16 q4 (16.7 / 17.6 at 4096 x 14336), for q8 pairs (34.3 /
-  // 45.4) and where tiles are many (fp16 q4 128256 x 4096 68 / 96).
+  // us: q8 fp16 at 8 rows 6144 x 4096 11.2 / 13.0, 14336 x 4096 19.5 / 19.7; bf16
+  // q4 at 4 rows 8192 x 4096 9.3 / 9.8, 16384 x 4096 14.7 / 14.9, 2 x 8192 x 2048
+  // 10.1 / 10.2.  The ring is ahead for fp16 q4 and q8 pairs, where tiles are
+  // many, and for bf16 q4 at 5-8 rows of more than two and a half tiles a CU
+  // (12288 x 4096 12.2 / 13.2, 4096 x 14336 17.9 / 19.4; 5120 x 5120 14.0 / 12.0).
   constexpr bool ONE = NMAT == 2 ? BITS == 4 && !__is_same(AT, f16) : BITS == 8 || !__is_same(AT, f16);
   if constexpr (ONE) {
-    if (a.M <= 8 && (int64_t)p.tiles * p.slices <= 4 * device_cu_count()) {
+    const int cus = device_cu_count();
+    if (a.M <= 8 && (int64_t)p.tiles * p.slices <= (BITS == 4 && NMAT == 1 && a.M > 4 ? 5 * cus / 2 : 4 * cus)) {
       if (a.M <= 4) return few_launch<BITS, AT, NMAT, 1, NMAT, LG, MAGIC, EPI, 4>(a, ws, st);
       return few_launch<BITS, AT, NMAT, 1, NMAT, LG, MAGIC, EPI, 8>(a, ws, st);
     }
   }
-  // the ring: no deeper than the run is long, and what the registers hold
-  // beside the activations
+  // The ring: a turn of one tile for pairs and for short odd runs, of two for
+  // other runs.  What a turn holds past the run's end is fetched and multiplied
+  // for nothing.  us at 5 rows of q4 fp16, turns of 1 / 2 / 4 tiles: 12288 x 4096
+  // (runs of 3) 10.5 / 12.1 / 13.5, 20480 x 4096 (5) 15.1 / 15.7 / 19.7, 4096 x
+  // 14336 (4 a slice) 14.9 / 14.8 / 16.6, 128256 x 4096 72 / 68 / 69; the pair 2 x
+  // 11008 x 4096 with one tile 15.8, with two 19.4.
+  const bool odd = (run & 1) && run <= 5;
   if (a.M <= 16) {
-    if constexpr (BITS == 4) {
-      if (run * NMAT > 2) return few_launch<BITS, AT, NMAT, 1, 4, LG, MAGIC, EPI, 0>(a, ws, st);
-    }
-    if (NMAT == 2 || run > 1) return few_launch<BITS, AT, NMAT, 1, 2, LG, MAGIC, EPI, 0>(a, ws, st);
-    if constexpr (NMAT == 1) return few_launch<BITS, AT, NMAT, 1, 1, LG, MAGIC, EPI, 0>(a, ws, st);
+    if constexpr (NMAT == 1)
+      if (odd) return few_launch<BITS, AT, NMAT, 1, 1, LG, MAGIC, EPI, 0>(a, ws, st);
+    return few_launch<BITS, AT, NMAT, 1, 2, LG, MAGIC, EPI, 0>(a, ws, st);
   }
   if constexpr (BITS == 4) {
-    if constexpr (NMAT == 1) {
-      if (run > 2) return few_launch<BITS, AT, NMAT, 2, 3, LG, MAGIC, EPI, 0>(a, ws, st);
-      if (run == 1) return few_launch<BITS, AT, NMAT, 2, 1, LG, MAGIC, EPI, 0>(a, ws, st);
-    }
+    if constexpr (NMAT == 1)
+      if (odd) return few_launch<BITS, AT, NMAT, 2, 1, LG, MAGIC, EPI, 0>(a, ws, st);
     return few_launch<BITS, AT, NMAT, 2, 2, LG, MAGIC, EPI, 0>(a, ws, st);
   }
   return MK_ERR_UNSUPPORTED;
