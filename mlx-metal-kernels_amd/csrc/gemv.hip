@@ -1318,7 +1318,8 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
   // 17-32 rows takes 6.5 us + 0.14 ns per 1000 weights for q4 fp16, 6.3 + 0.175
   // for bf16, and 3.3 for the sum of K slices).  17-32 rows over 8-bit codes: the
   // product for gate/up (2 x 14336 x 4096 40 us, two passes 66, the tile kernel
-  // 65), two passes for bf16 (44 against 65 at 4096 x 14336), the tile kernel
+  // 65) unless its workgroups are few (2 x 4096 x 4096: 23.6, the tile kernel
+  // 18.8), two passes for bf16 (44 against 65 at 4096 x 14336), the tile kernel
   // below for fp16.
   {
     constexpr int64_t kPass = BITS == 4 ? 32 : 16;
@@ -1326,14 +1327,31 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
                      (EPI != EPI_ROPE_KV || act_dt == MK_DT_F16) &&
                      few_ok<BITS, NMAT>(a, M < kPass ? M : kPass, gs, sc_dt, ws_bytes);
     const bool wide8 = BITS == 8 && M > kPass;
+    const bool few_rest = M > 32 && M <= 48 && few_ok<BITS, NMAT>(a, M - 32, gs, sc_dt, ws_bytes);
     if constexpr (EPI != EPI_ROPE_KV) {
       bool product = (M >= product_rows || (wide8 && NMAT == 2)) && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
-      if (product && few && M <= kPass) {
+      if (BITS == 8 && product && M < kGemmMinRows && tile_eligible<NMAT>(a, act_dt, sc_dt)) {
+        const float more = 2.0f * (float)N * (float)K - 3.3e7f;  // weights past those that take one round
+        product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 18.0f + (more > 0.0f ? 5.6e-7f * more : 0.0f);
+      } else if (product && few && M <= kPass) {
         product = false;  // one pass
       } else if (product && few && M >= kGemmMinRows && BITS == 4 && NMAT == 1) {
         const float weights = (float)N * (float)K, sum = K > 4096 ? 3.3f : 0.0f;
         const float pass = act_dt == MK_DT_F16 ? 6.5f + 1.4e-7f * weights + sum : 6.3f + 1.75e-7f * weights + sum;
         product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 2.0f * pass;
+      }
+      if (BITS == 8 && NMAT == 1 && product && few_rest && tile_eligible<NMAT>(a, act_dt, sc_dt)) {
+        // 33-48 rows: the tile kernel (2.7 us + 0.66 ns per 1000 weights) and a
+        // few-row pass (5 + 0.25, 3.3 for the sum) where the product's workgroups
+        // are few: 4096 x 14336 at 40 rows 64 us against 70.  (Its estimate, of
+        // 4-bit codes, is 10-15 % high here.)
+        const float weights = (float)N * (float)K;
+        if (7.7f + 9.1e-7f * weights + (K > 4096 ? 3.3f : 0.0f) < 0.85f * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K)) {
+          rc = gemv_dispatch<BITS, NMAT, EPI>(a, 32, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes);
+          GemvArgs b = a;
+          rows_from(b, 32);
+          return rc != MK_OK ? rc : gemv_dispatch<BITS, NMAT, EPI>(b, M - 32, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes);
+        }
       }
       if (product) {
         GemvArgs b = a;
