@@ -412,8 +412,11 @@ inline int kv_group_chunks_log2(int64_t D, int64_t gs) {
   return __builtin_ctzll((unsigned long long)l);
 }
 
-// chunks of 256 threads per launch: far below the grid limit of 2^31 - 1
-constexpr int64_t kMaxKvChunks = (int64_t)256 << 30;
+// A launch of the vector kernels, a thread per chunk in blocks of 256, is under
+// 2^32 threads (HIP's limit for a grid's dimension): 2^35 values, 64 GiB of fp16.
+// The other kernels take a thread per row, or stride over the grid.
+constexpr int64_t kMaxKvChunks = ((int64_t)1 << 32) - 256;
+static_assert((kMaxKvChunks + 255) / 256 * 256 < ((int64_t)1 << 32), "threads of the largest launch");
 
 }  // namespace
 
