@@ -1319,8 +1319,9 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
   // for bf16, and 3.3 for the sum of K slices).  17-32 rows over 8-bit codes: the
   // product for gate/up (2 x 14336 x 4096 40 us, two passes 66, the tile kernel
   // 65) unless its workgroups are few (2 x 4096 x 4096: 23.6, the tile kernel
-  // 18.8), two passes for bf16 (44 against 65 at 4096 x 14336), the tile kernel
-  // below for fp16.
+  // 18.8), two passes for bf16 (44 against 65 at 4096 x 14336) and for fp16
+  // where the tile kernel does not apply (4096 x 4064 19.0 against 23.2; not with
+  // K slices: 4096 x 4128 25.6 against 24.4), else the kernels below.
   {
     constexpr int64_t kPass = BITS == 4 ? 32 : 16;
     const bool few = M <= 2 * kPass && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
@@ -1359,7 +1360,7 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
         return launch_gemm_rows<BITS, NMAT, NMAT == 1 ? EPI_RESIDUAL : EPI>(b, act_dt, sc_dt, st);
       }
     }
-    if (few && !(wide8 && act_dt == MK_DT_F16)) {
+    if (few && !(wide8 && act_dt == MK_DT_F16 && (tile_eligible<NMAT>(a, act_dt, sc_dt) || K > 4096))) {
       for (int64_t m0 = 0; m0 < M && rc == MK_OK; m0 += kPass) {
         GemvArgs b = a;
         b.M = (int)(M - m0 < kPass ? M - m0 : kPass);
