@@ -402,20 +402,27 @@ __global__ __launch_bounds__(256) void gemv_slices_kernel(const GemvArgs args, c
 struct FewPlan {
   int slices, nw, runs, tiles;
 };
+// K slices of at most FMAXW waves, and the workgroups of a slice: a CU's eight
+// waves are one workgroup or, where rows are short, several.  (One a CU, then
+// this, us at 8 rows of 33000 x 1024: q4 fp16 13.2 -> 7.9, bf16 18.0 -> 9.4, q8
+// fp16 15.3 -> 10.6.  Pairs of 8-bit codes keep half of the waves idle rather
+// than double them: 2 x 8192 x 2048 11.9, 12.4 with two workgroups.)
+template <int BITS, int NMAT>
 inline FewPlan few_plan(int N, int K, int cus) {
   FewPlan p;
   const int waves = (K + FKW - 1) / FKW;
   p.slices = (waves + FMAXW - 1) / FMAXW;
   p.nw = (waves + p.slices - 1) / p.slices;
   p.tiles = (N + 15) / 16;
-  const int runs = cus / p.slices > 0 ? cus / p.slices : 1;
+  const int groups = cus * (BITS == 8 && NMAT == 2 && p.nw > 2 ? 1 : FMAXW / p.nw);
+  const int runs = groups / p.slices > 0 ? groups / p.slices : 1;
   p.runs = p.tiles < runs ? p.tiles : runs;
   return p;
 }
 
 template <int BITS, typename AT, int NMAT, int MT, int DU, int LG, bool MAGIC, int EPI, int XL>
 int few_launch(const GemvArgs& a, float* ws, hipStream_t st) {
-  FewPlan p = few_plan(a.N, a.K, device_cu_count());
+  FewPlan p = few_plan<BITS, NMAT>(a.N, a.K, device_cu_count());
   if (XL) p.runs = p.tiles;
   FewArgs f;
   f.g = a;
@@ -437,19 +444,20 @@ int few_launch(const GemvArgs& a, float* ws, hipStream_t st) {
 
 template <int BITS, typename AT, int NMAT, int EPI, int LG, bool MAGIC = __is_same(AT, f16)>
 int few_columns(const GemvArgs& a, float* ws, hipStream_t st) {
-  const FewPlan p = few_plan(a.N, a.K, device_cu_count());
+  const FewPlan p = few_plan<BITS, NMAT>(a.N, a.K, device_cu_count());
   const int run = (p.tiles + p.runs - 1) / p.runs;  // tiles of the longest run
   // Up to 8 rows of the forms whose unpacking weighs most, while tiles are
   // few: one tile per workgroup (XL), two workgroups a CU.  Against the ring,
   // us: q8 fp16 at 8 rows 6144 x 4096 11.2 / 13.0, 14336 x 4096 19.5 / 19.7; bf16
   // q4 at 4 rows 8192 x 4096 9.3 / 9.8, 16384 x 4096 14.7 / 14.9, 2 x 8192 x 2048
   // 10.1 / 10.2.  The ring is ahead for fp16 q4 and q8 pairs, where tiles are
-  // many, and for bf16 q4 at 5-8 rows of more than two and a half tiles a CU
-  // (12288 x 4096 12.2 / 13.2, 4096 x 14336 17.9 / 19.4; 5120 x 5120 14.0 / 12.0).
+  // many, and for bf16 q4 at 5-8 rows of more than 20 waves a CU (12288 x 4096
+  // 12.2 / 13.2, 4096 x 14336 17.9 / 19.4; 5120 x 5120 14.0 / 12.0).
   constexpr bool ONE = NMAT == 2 ? BITS == 4 && !__is_same(AT, f16) : BITS == 8 || !__is_same(AT, f16);
   if constexpr (ONE) {
-    const int cus = device_cu_count();
-    if (a.M <= 8 && (int64_t)p.tiles * p.slices <= (BITS == 4 && NMAT == 1 && a.M > 4 ? 5 * cus / 2 : 4 * cus)) {
+    const int64_t ones = (int64_t)p.tiles * p.slices, cus = device_cu_count();
+    const bool few_waves = BITS == 8 || NMAT == 2 || a.M <= 4 || ones * p.nw <= 20 * cus;
+    if (a.M <= 8 && ones <= 4 * cus && few_waves) {
       if (a.M <= 4) return few_launch<BITS, AT, NMAT, 1, NMAT, LG, MAGIC, EPI, 4>(a, ws, st);
       return few_launch<BITS, AT, NMAT, 1, NMAT, LG, MAGIC, EPI, 8>(a, ws, st);
     }
@@ -500,7 +508,7 @@ namespace mkq {
 size_t few_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M > 32 && M <= 68) M = 32;  // two passes (and up to 4 rows past them)
   if (M < 1 || M > 32 || N < 1 || K < 1 || N >= (1LL << 26) || K >= (1LL << 26)) return 0;
-  const FewPlan p = few_plan((int)N, (int)K, device_cu_count());
+  const FewPlan p = few_plan<4, 1>((int)N, (int)K, device_cu_count());  // (slices do not depend on the form)
   return p.slices > 1 ? (size_t)p.slices * M * N * sizeof(float) : 0;
 }
 
