@@ -1250,6 +1250,21 @@ inline int dot_waves(int64_t K) {
 // up to 32 rows through the kernels here)
 constexpr int64_t kGemmMinRows = 33;
 
+// Estimated us of the tile kernel's 17-32 rows: rounds of workgroups over the
+// CUs, each as long as a row.  Measured at 32 rows (17 rows), this in brackets,
+// q8: 4096 x 4096 13.8 (11.3) [13.9 (10.5)], 6144 x 4096 24.6 (19.2) [24.8
+// (18.0)], 4096 x 14336 41.4 (32.1) [41.1 (29.6)], 33000 x 1024 27.7 [27.5], 2 x
+// 4096 x 4096 18.9 (16.4) [18.6 (16.4)], 2 x 14336 x 4096 65.4 (55.0) [65.4
+// (56.7)]; q4: 2 x 8192 x 8192 55.2 [55.2].
+template <int BITS, int NMAT>
+inline float tile_rows_us(int64_t M, int64_t N, int64_t K) {
+  const int cus = device_cu_count();
+  const float rounds = (float)(((N + 15) / 16 + cus - 1) / cus);
+  const float us = BITS == 4 ? 3.26f : NMAT == 2 ? 3.9f : 2.72f;  // per 1024 k
+  const float rows = NMAT == 2 ? 0.7f + 0.0094f * (float)M : 0.53f + 0.0147f * (float)M;
+  return 3.0f + rounds * us * rows * (float)K / 1024.0f;
+}
+
 // Rows of a whole pass: the 1-4 rows (q8: 2) that a batch leaves past its last
 // one take the v_dot2 kernel, which does not round W, as when every batch ran in
 // passes.  (16 where two column tiles' partial sums and a pair's 128 groups of
@@ -1302,7 +1317,7 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
       // us at 33 / 36 / 65 rows, all rows in one form -> this, q4 g64:
       // 2 x 14336 x 4096 36 / 35 / 53 -> 35 / 42 / 47, 6144 x 4096 18 / 18 / 22
       // -> 16 / 18 / 26, 4096 x 14336 35 / 36 / 67 -> 28 / 32 / 48
-      rc = gemv_dispatch<BITS, NMAT, EPI>(a, M - tail, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes, BITS == 4 ? 32 : 33);
+      rc = gemv_dispatch<BITS, NMAT, EPI>(a, M - tail, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes, BITS == 4 && NMAT == 2 ? 32 : 33);
       if (rc != MK_OK) return rc;
       GemvArgs b = a;
       b.M = (int)tail;
@@ -1316,12 +1331,13 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
   // rows, unless two passes take less: few output rows over a long K leave the
   // product 64 workgroups (4096 x 14336 at 40 rows 66 us against 34; a pass of
   // 17-32 rows takes 6.5 us + 0.14 ns per 1000 weights for q4 fp16, 6.3 + 0.175
-  // for bf16, and 3.3 for the sum of K slices).  17-32 rows over 8-bit codes: the
-  // product for gate/up (2 x 14336 x 4096 40 us, two passes 66, the tile kernel
-  // 65) unless its workgroups are few (2 x 4096 x 4096: 23.6, the tile kernel
-  // 18.8), two passes for bf16 (44 against 65 at 4096 x 14336) and for fp16
-  // where the tile kernel does not apply (4096 x 4064 19.0 against 23.2; not with
-  // K slices: 4096 x 4128 25.6 against 24.4), else the kernels below.
+  // for bf16, and 3.3 for the sum of K slices).  17-32 rows over 8-bit codes, fp16:
+  // the product or the tile kernel below, whichever is estimated to take less (2
+  // x 14336 x 4096 at 32 rows 40 us and 65, 2 x 4096 x 4096 23.3 and 18.9, 33000 x
+  // 1024 23.2 and 27.7), and two passes where neither applies (4096 x 4064 19.0,
+  // the MFMA kernel 23.2; not with K slices: 4096 x 4128 25.6 against 24.4).  bf16:
+  // the product for pairs (two passes 66), two passes for one matrix (4096 x
+  // 14336 44 against 78).
   {
     constexpr int64_t kPass = BITS == 4 ? 32 : 16;
     const bool few = M <= 2 * kPass && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
@@ -1330,10 +1346,10 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
     const bool wide8 = BITS == 8 && M > kPass;
     const bool few_rest = M > 32 && M <= 48 && few_ok<BITS, NMAT>(a, M - 32, gs, sc_dt, ws_bytes);
     if constexpr (EPI != EPI_ROPE_KV) {
-      bool product = (M >= product_rows || (wide8 && NMAT == 2)) && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
-      if (BITS == 8 && product && M < kGemmMinRows && tile_eligible<NMAT>(a, act_dt, sc_dt)) {
-        const float more = 2.0f * (float)N * (float)K - 3.3e7f;  // weights past those that take one round
-        product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 18.0f + (more > 0.0f ? 5.6e-7f * more : 0.0f);
+      const bool tile = tile_eligible<NMAT>(a, act_dt, sc_dt);
+      bool product = (M >= product_rows || (wide8 && (NMAT == 2 || tile))) && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
+      if (product && M < kGemmMinRows && tile && !(BITS == 4 && few)) {
+        product = 0.9f * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < tile_rows_us<BITS, NMAT>(M, N, K);
       } else if (product && few && M <= kPass) {
         product = false;  // one pass
       } else if (product && few && M >= kGemmMinRows && BITS == 4 && NMAT == 1) {
@@ -1341,13 +1357,12 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
         const float pass = act_dt == MK_DT_F16 ? 6.5f + 1.4e-7f * weights + sum : 6.3f + 1.75e-7f * weights + sum;
         product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 2.0f * pass;
       }
-      if (BITS == 8 && NMAT == 1 && product && few_rest && tile_eligible<NMAT>(a, act_dt, sc_dt)) {
-        // 33-48 rows: the tile kernel (2.7 us + 0.66 ns per 1000 weights) and a
-        // few-row pass (5 + 0.25, 3.3 for the sum) where the product's workgroups
-        // are few: 4096 x 14336 at 40 rows 64 us against 70.  (Its estimate, of
-        // 4-bit codes, is 10-15 % high here.)
-        const float weights = (float)N * (float)K;
-        if (7.7f + 9.1e-7f * weights + (K > 4096 ? 3.3f : 0.0f) < 0.85f * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K)) {
+      if (BITS == 8 && NMAT == 1 && product && few_rest && tile) {
+        // 33-48 rows: the tile kernel and a few-row pass (4.5 us + 0.24 ns per
+        // 1000 weights, 3.3 for the sum of K slices) where the product's
+        // workgroups are few: 4096 x 14336 at 40 rows 63 us against 70
+        const float pass = 4.5f + 2.4e-7f * (float)N * (float)K + (K > 4096 ? 3.3f : 0.0f);
+        if (tile_rows_us<BITS, NMAT>(32, N, K) + pass < 0.85f * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K)) {
           rc = gemv_dispatch<BITS, NMAT, EPI>(a, 32, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes);
           GemvArgs b = a;
           rows_from(b, 32);
