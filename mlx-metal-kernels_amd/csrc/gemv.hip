@@ -1340,7 +1340,13 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
   // 14336 44 against 78).
   {
     constexpr int64_t kPass = BITS == 4 ? 32 : 16;
-    const bool few = M <= 2 * kPass && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
+    const int64_t tiles = (N + 15) / 16, cus = device_cu_count();
+    // 5-12 rows of long rows on one round of the K-split kernel: no sum of slices
+    // (4096 x 8192 at 6 rows 10.6 against 11.5, 4096 x 11008 14.0 against 18.3;
+    // 4096 x 14336 15.2 against 15.1, two rounds 5120 x 8192 18.2 against 13.0)
+    const bool ksplit = NMAT == 1 && K > 4096 && M >= kXkMinRows && M <= (K <= 11264 ? 12 : K <= 12288 ? 8 : 0) &&
+                        tiles <= cus && 2 * tiles > cus && xk_eligible<BITS, NMAT>(a, 1, act_dt, sc_dt);
+    const bool few = M <= 2 * kPass && !ksplit && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
                      (EPI != EPI_ROPE_KV || act_dt == MK_DT_F16) &&
                      few_ok<BITS, NMAT>(a, M < kPass ? M : kPass, gs, sc_dt, ws_bytes);
     const bool wide8 = BITS == 8 && M > kPass;
