@@ -445,18 +445,21 @@ int few_launch(const GemvArgs& a, float* ws, hipStream_t st) {
 template <int BITS, typename AT, int NMAT, int EPI, int LG, bool MAGIC = __is_same(AT, f16)>
 int few_columns(const GemvArgs& a, float* ws, hipStream_t st) {
   const FewPlan p = few_plan<BITS, NMAT>(a.N, a.K, device_cu_count());
-  const int run = (p.tiles + p.runs - 1) / p.runs;  // tiles of the longest run
+  // tiles of a run: the longest, unless few are that long (4096 x 11008: 85 runs
+  // of three slices, one of them 4 tiles, the others 3)
+  const int run = p.tiles / p.runs + (4 * (p.tiles % p.runs) >= p.runs ? 1 : 0);
   // Up to 8 rows of the forms whose unpacking weighs most, while tiles are
   // few: one tile per workgroup (XL), two workgroups a CU.  Against the ring,
   // us: q8 fp16 at 8 rows 6144 x 4096 11.2 / 13.0, 14336 x 4096 19.5 / 19.7; bf16
   // q4 at 4 rows 8192 x 4096 9.3 / 9.8, 16384 x 4096 14.7 / 14.9, 2 x 8192 x 2048
   // 10.1 / 10.2.  The ring is ahead for fp16 q4 and q8 pairs, where tiles are
   // many, and for bf16 q4 at 5-8 rows of more than 20 waves a CU (12288 x 4096
-  // 12.2 / 13.2, 4096 x 14336 17.9 / 19.4; 5120 x 5120 14.0 / 12.0).
+  // 12.2 / 13.2, 4096 x 14336 17.9 / 19.4; 5120 x 5120 14.0 / 12.0) unless scales
+  // come one by one (4096 x 11008 16.6 / 18.6).
   constexpr bool ONE = NMAT == 2 ? BITS == 4 && !__is_same(AT, f16) : BITS == 8 || !__is_same(AT, f16);
   if constexpr (ONE) {
     const int64_t ones = (int64_t)p.tiles * p.slices, cus = device_cu_count();
-    const bool few_waves = BITS == 8 || NMAT == 2 || a.M <= 4 || ones * p.nw <= 20 * cus;
+    const bool few_waves = BITS == 8 || NMAT == 2 || a.M <= 4 || LG == 0 || ones * p.nw <= 20 * cus;
     if (a.M <= 8 && ones <= 4 * cus && few_waves) {
       if (a.M <= 4) return few_launch<BITS, AT, NMAT, 1, NMAT, LG, MAGIC, EPI, 4>(a, ws, st);
       return few_launch<BITS, AT, NMAT, 1, NMAT, LG, MAGIC, EPI, 8>(a, ws, st);
