@@ -1346,7 +1346,21 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
     // 4096 x 14336 15.2 against 15.1, two rounds 5120 x 8192 18.2 against 13.0)
     const bool ksplit = NMAT == 1 && K > 4096 && M >= kXkMinRows && M <= (K <= 11264 ? 12 : K <= 12288 ? 8 : 0) &&
                         tiles <= cus && 2 * tiles > cus && xk_eligible<BITS, NMAT>(a, 1, act_dt, sc_dt);
-    const bool few = M <= 2 * kPass && !ksplit && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
+    // rows of more than 4096 k, not in whole 512s (the few-row kernel's slices are
+    // uneven there and its scales come one by one): up to 8 rows by the MFMA kernel,
+    // which has no sum of slices (q4 fp16 at 5 rows 4096 x 11008 13.6 against 16.3,
+    // 4096 x 5056 9.5 against 11.2, 3072 x 9984 12.1 against 13.7, but 1024 x 11008
+    // 12.5 against 9.4; q8 4096 x 11008 18.1 against 20.1, 4096 x 8256 17.3 against
+    // 16.9; bf16 q4 16.5 against 16.1)
+    const bool uneven = NMAT == 1 && fast && K > 4096 && K % 512 != 0 && M <= 8 && 2 * tiles > cus &&
+                        (BITS == 4 ? act_dt == MK_DT_F16 : K > 10240);
+    // short rows of few outputs: the few-row kernel's waves have 512 k each, the
+    // kernels below share a row among more (2048 x 512, us: q4 fp16 at 17 rows 3.2
+    // against 4.6, q8 fp16 at 8 rows 3.3 against 4.0, q8 bf16 at 32 rows 6.6 against
+    // 8.6; 2 x 2048 x 512 q4 fp16 at 17 rows 4.3 against 6.3; 2 x 8192 x 512 bf16 6.9
+    // against 6.0)
+    const bool brief = fast && K <= 512 && tiles <= 128 && (BITS == 8 || act_dt == MK_DT_F16 ? M <= 32 : M <= 16);
+    const bool few = M <= 2 * kPass && !ksplit && !uneven && !brief && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
                      (EPI != EPI_ROPE_KV || act_dt == MK_DT_F16) &&
                      few_ok<BITS, NMAT>(a, M < kPass ? M : kPass, gs, sc_dt, ws_bytes);
     const bool wide8 = BITS == 8 && M > kPass;
@@ -1355,7 +1369,9 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
       const bool tile = tile_eligible<NMAT>(a, act_dt, sc_dt);
       bool product = (M >= product_rows || (wide8 && (NMAT == 2 || tile))) && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
       if (product && M < kGemmMinRows && tile && !(BITS == 4 && few)) {
-        product = 0.9f * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < tile_rows_us<BITS, NMAT>(M, N, K);
+        // (short rows: the estimate leaves out what every workgroup takes to start)
+        const float us = (K <= 1024 ? 1.25f : 0.9f) * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K);
+        product = us < tile_rows_us<BITS, NMAT>(M, N, K);
       } else if (product && few && M <= kPass) {
         product = false;  // one pass
       } else if (product && few && M >= kGemmMinRows && BITS == 4 && NMAT == 1) {

@@ -17,7 +17,7 @@ CASES = [  # M, N, K
     (5, 1, 32), (8, 15, 96), (9, 33, 544), (16, 100, 512), (17, 257, 1056), (32, 600, 2080),
     # several tiles per workgroup (ring refills, turns of one tile and of two, a last partial turn); K slices of 4096 and less, the last partly past K
     (6, 9000, 1024), (31, 17000, 512), (7, 1000, 4128), (16, 515, 14336), (32, 4096, 8224), (20, 5000, 4608),
-    (40, 4096, 14336), (33, 700, 5120), (28, 700, 4128), (7, 3072, 8192), (12, 4096, 6144), (9, 25000, 512), (20, 25000, 512)]
+    (40, 4096, 14336), (33, 700, 5120), (28, 700, 4128), (7, 3072, 8192), (12, 4096, 6144), (8, 3000, 5056), (5, 2100, 11008), (9, 25000, 512), (20, 25000, 512)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
