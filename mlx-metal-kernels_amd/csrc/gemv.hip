@@ -1341,10 +1341,13 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
   {
     constexpr int64_t kPass = BITS == 4 ? 32 : 16;
     const int64_t tiles = (N + 15) / 16, cus = device_cu_count();
-    // 5-12 rows of long rows on one round of the K-split kernel: no sum of slices
-    // (4096 x 8192 at 6 rows 10.6 against 11.5, 4096 x 11008 14.0 against 18.3;
-    // 4096 x 14336 15.2 against 15.1, two rounds 5120 x 8192 18.2 against 13.0)
-    const bool ksplit = NMAT == 1 && K > 4096 && M >= kXkMinRows && M <= (K <= 11264 ? 12 : K <= 12288 ? 8 : 0) &&
+    // a few of the batch sizes on one round of the K-split kernel, which has no sum
+    // of slices (4096 x 6144 at 8 rows 9.2 against 10.5, at 16 10.6 against 10.9; 4096
+    // x 8192 at 6 10.6 against 11.5, at 12 11.8 against 11.9; 2560 x 6912, not in
+    // whole 512s, at 17 12.9 against 14.4; 4096 x 14336 at 6 15.2 against 15.1; two
+    // rounds 5120 x 8192 at 6 18.2 against 13.0)
+    const int64_t most = K > 12288 ? 0 : K % 512 != 0 ? 20 : K <= 6144 ? 16 : K <= 11264 ? 12 : 8;
+    const bool ksplit = NMAT == 1 && K > 4096 && M >= kXkMinRows && M <= most &&
                         tiles <= cus && 2 * tiles > cus && xk_eligible<BITS, NMAT>(a, 1, act_dt, sc_dt);
     // rows of more than 4096 k, not in whole 512s (the few-row kernel's slices are
     // uneven there and its scales come one by one): up to 8 rows by the MFMA kernel,
@@ -1358,8 +1361,10 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
     // kernels below share a row among more (2048 x 512, us: q4 fp16 at 17 rows 3.2
     // against 4.6, q8 fp16 at 8 rows 3.3 against 4.0, q8 bf16 at 32 rows 6.6 against
     // 8.6; 2 x 2048 x 512 q4 fp16 at 17 rows 4.3 against 6.3; 2 x 8192 x 512 bf16 6.9
-    // against 6.0)
-    const bool brief = fast && K <= 512 && tiles <= 128 && (BITS == 8 || act_dt == MK_DT_F16 ? M <= 32 : M <= 16);
+    // against 6.0; 2 x 4864 x 896 at 17 rows 7.2 against 8.9)
+    const bool brief = fast && ((K <= 512 && tiles <= 128 && (BITS == 8 || act_dt == MK_DT_F16 ? M <= 32 : M <= 16)) ||
+                                (NMAT == 2 && K < 1024 && K % 512 != 0 && M >= 17 && M <= 32 &&
+                                 tile_eligible<NMAT>(a, act_dt, sc_dt)));
     const bool few = M <= 2 * kPass && !ksplit && !uneven && !brief && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
                      (EPI != EPI_ROPE_KV || act_dt == MK_DT_F16) &&
                      few_ok<BITS, NMAT>(a, M < kPass ? M : kPass, gs, sc_dt, ws_bytes);
@@ -1380,11 +1385,12 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
         product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 2.0f * pass;
       }
       if (BITS == 8 && NMAT == 1 && product && few_rest && tile) {
-        // 33-48 rows: the tile kernel and a few-row pass (4.5 us + 0.24 ns per
+        // 33-48 rows: the tile kernel and a few-row pass (5.2 us + 0.24 ns per
         // 1000 weights, 3.3 for the sum of K slices) where the product's
-        // workgroups are few: 4096 x 14336 at 40 rows 63 us against 70
-        const float pass = 4.5f + 2.4e-7f * (float)N * (float)K + (K > 4096 ? 3.3f : 0.0f);
-        if (tile_rows_us<BITS, NMAT>(32, N, K) + pass < 0.85f * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K)) {
+        // workgroups are few: 4096 x 14336 at 40 rows 63 us against 70, 4096 x
+        // 8192 37 against 40, 2048 x 2048 13.4 against 12.1
+        const float pass = 5.2f + 2.4e-7f * (float)N * (float)K + (K > 4096 ? 3.3f : 0.0f);
+        if (tile_rows_us<BITS, NMAT>(32, N, K) + pass < 0.9f * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K)) {
           rc = gemv_dispatch<BITS, NMAT, EPI>(a, 32, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes);
           GemvArgs b = a;
           rows_from(b, 32);
