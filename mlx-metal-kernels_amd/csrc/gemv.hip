@@ -1385,11 +1385,11 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
         product = gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K) < 2.0f * pass;
       }
       if (BITS == 8 && NMAT == 1 && product && few_rest && tile) {
-        // 33-48 rows: the tile kernel and a few-row pass (5.2 us + 0.24 ns per
+        // 33-48 rows: the tile kernel and a few-row pass (5-6 us + 0.24 ns per
         // 1000 weights, 3.3 for the sum of K slices) where the product's
         // workgroups are few: 4096 x 14336 at 40 rows 63 us against 70, 4096 x
-        // 8192 37 against 40, 2048 x 2048 13.4 against 12.1
-        const float pass = 5.2f + 2.4e-7f * (float)N * (float)K + (K > 4096 ? 3.3f : 0.0f);
+        // 11008 50 against 67, but 2048 x 2048 13.4 against 12.1
+        const float pass = 4.9f + 0.07f * (float)(M - 32) + 2.4e-7f * (float)N * (float)K + (K > 4096 ? 3.3f : 0.0f);
         if (tile_rows_us<BITS, NMAT>(32, N, K) + pass < 0.9f * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K)) {
           rc = gemv_dispatch<BITS, NMAT, EPI>(a, 32, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes);
           GemvArgs b = a;
