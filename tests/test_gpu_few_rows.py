@@ -9,15 +9,18 @@ import torch
 
 import mk.quant_ops as qo
 from mk import _lib
-from tests.test_gpu_gemm_rows import _check, _check_rows, _rounded, _weight
+from tests.test_gpu_gemm_rows import HALF_ULP, _check, _check_rows, _rounded, _weight
 
 pytestmark = pytest.mark.gpu
 
 CASES = [  # M, N, K
-    (5, 1, 32), (8, 15, 96), (9, 33, 544), (16, 100, 512), (17, 257, 1056), (32, 600, 2080),
-    # several tiles per workgroup (ring refills, turns of one tile and of two, a last partial turn); K slices of 4096 and less, the last partly past K
+    (5, 1, 32), (8, 15, 96), (9, 33, 544), (16, 100, 512), (16, 3000, 512), (17, 257, 1056), (32, 600, 2080),
+    # several tiles per workgroup (ring refills, turns of one tile and of two, a last partial turn); K slices of 4096
+    # and less, the last partly past K
     (6, 9000, 1024), (31, 17000, 512), (7, 1000, 4128), (16, 515, 14336), (32, 4096, 8224), (20, 5000, 4608),
-    (40, 4096, 14336), (33, 700, 5120), (28, 700, 4128), (7, 3072, 8192), (12, 4096, 6144), (8, 3000, 5056), (5, 2100, 11008), (9, 25000, 512), (20, 25000, 512)]
+    (40, 4096, 14336), (33, 700, 5120), (28, 700, 4128), (9, 25000, 512), (20, 25000, 512),
+    # rows that go to the K-split and MFMA kernels in fp16
+    (7, 3072, 8192), (12, 4096, 6144), (8, 3000, 5056), (5, 2100, 11008)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -27,7 +30,7 @@ def test_few_rows(dev, M, N, K, bits, dtype):
     gen = torch.Generator(device=dev).manual_seed(M * 7 + N + K)
     x = torch.randn((M, K), generator=gen, device=dev).to(dtype)
     fn = qo.q4_matvec_decode if bits == 4 else qo.q8_matvec_decode
-    for g, zeros in ((64, "whole"), (32, "whole"), (128, "none"), (256, "whole")):
+    for g, zeros in ((64, "whole"), (32, "whole"), (128, "whole"), (256, "whole"), (128, "none"), (64, "affine")):
         codes, packed, s, z = _weight(gen, dev, N, K, bits, g, torch.float16, zeros)
         got = fn(x, packed, s, z, group_size=g)
         _check_rows(got, x, codes, s, z, g, bits, f"M{M} N{N} K{K} q{bits} g{g} {zeros}")
@@ -37,17 +40,23 @@ def test_few_rows(dev, M, N, K, bits, dtype):
         assert torch.equal(out, (res.float() + mm.float()).to(dtype))
 
 
+@pytest.mark.parametrize("g", [32, 64, 128, 256])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("M,N,K", [(5, 7, 64), (8, 300, 1024), (12, 14336, 512), (32, 9000, 1024), (24, 100, 4096)])
-def test_few_rows_gate_up(dev, M, N, K, bits, dtype):
+@pytest.mark.parametrize("M,N,K", [(5, 7, 64), (8, 300, 1024), (12, 14336, 512), (32, 9000, 1024), (24, 100, 4096), (16, 3000, 1056)])
+def test_few_rows_gate_up(dev, M, N, K, bits, dtype, g):
     gen = torch.Generator(device=dev).manual_seed(M + N + K)
     x = torch.randn((M, K), generator=gen, device=dev).to(dtype)
-    cg, gw, gs, gz = _weight(gen, dev, N, K, bits, 64, torch.float16, "whole")
-    cu, uw, us, uz = _weight(gen, dev, N, K, bits, 64, torch.float16, "whole")
-    gate, up, _ = qo.q_gate_up_swiglu(x, gw, uw, gs, us, gz, uz, bits=bits, group_size=64, return_gate_up=True)
-    _check(gate, x, _rounded(cg, gs, gz, 64, dtype), dtype, "gate")
-    _check(up, x, _rounded(cu, us, uz, 64, dtype), dtype, "up")
+    for zeros in ("whole", "affine"):
+        cg, gw, gs, gz = _weight(gen, dev, N, K, bits, g, torch.float16, zeros)
+        cu, uw, us, uz = _weight(gen, dev, N, K, bits, g, torch.float16, zeros)
+        gate, up, mlp = qo.q_gate_up_swiglu(x, gw, uw, gs, us, gz, uz, bits=bits, group_size=g, return_gate_up=True)
+        _check_rows(gate, x, cg, gs, gz, g, bits, ("gate", zeros))
+        _check_rows(up, x, cu, us, uz, g, bits, ("up", zeros))
+        gf = gate.double()
+        want = gf / (1 + torch.exp(-gf)) * up.double()
+        # silu in fp32 (a few 2^-24), the product rounded once
+        assert bool(((mlp.double() - want).abs() <= 1.01 * HALF_ULP[dtype] * want.abs() + 2.0 ** -24).all())
 
 
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
