@@ -101,7 +101,8 @@ int mk_q8_matvec(const void* x, const uint8_t* w, const void* scales, const void
  * mk_matvec_workspace_bytes(M, N, K) bytes: 0 unless M <= 68 and K > 4096,
  * where it lets passes of up to 32 rows split K over workgroups (the fp32 sums of the
  * slices go through it).  Without one such calls take the kernels that walk
- * whole rows. */
+ * whole rows, as gate/up pairs, the norm + matvec and the qkv + RoPE entries
+ * (which have no workspace argument) do for every K > 4096. */
 size_t mk_matvec_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int mk_q4_matvec_ws(const void* x, const uint8_t* w, const void* scales, const void* zeros, const void* residual,
                     void* y_mm, void* y_out, int64_t M, int64_t N, int64_t K, int64_t group_size, int act_dtype,

@@ -26,10 +26,11 @@
 // rows, for 256 CUs), the K slices fill the chip.
 //
 // Measured, q4 g64 fp16, us (passes of 32 rows before -> now): 509 rows
-// 2 x 14336 x 4096 + SwiGLU 428 -> 141 (850 TFLOP/s; 125 without the copies,
-// 115 without the unpacking) and 4096 x 14336 537 -> 100 (600; 67 without the
-// copies); 128 rows 109 -> 55 and 135 -> 67; 64 rows 57 -> 41 and 69 -> 67.
-// bf16 128 x 6144 x 4096 120 -> 27; q8 bf16 g32 300 x 32000 x 4096 1225 -> 162.
+// 2 x 14336 x 4096 + SwiGLU 428 -> 131 (915 TFLOP/s; as first built 141, 125
+// without the copies, 115 without the unpacking) and 4096 x 14336 537 -> 95 (630;
+// as first built 100, 67 without the copies); 128 rows 109 -> 52 and 135 -> 67; 64
+// rows 57 -> 35.  bf16 128 x 6144 x 4096 120 -> 26; q8 bf16 g32 300 x 32000 x 4096
+// 1225 -> 162.
 #include "common.h"
 #include "gemv_common.h"
 
@@ -402,7 +403,10 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2)
 // such a workgroup with every CU busy, measured (q4, fp16, groups of 64):
 // 2 x 14336 x 4096 at 509 rows 141 us as 8x8x1 (64 turns), 4096 x 14336 100 us
 // as 8x1x4 and 101 as 4x2x4 (56 turns), 2 x 14336 x 4096 at 128 rows 55 us as
-// 8x2x2 (32 turns), 4096 x 14336 at 64 rows 67 us as 4x1x4 (56 turns).
+// 8x2x2 (32 turns), 4096 x 14336 at 64 rows 67 us as 4x1x4 (56 turns).  The times
+// of this one type decide for all: bf16 takes 3-10 % longer, 8-bit codes 10-15 %
+// less where a turn is short and up to as much more where scales come one by one,
+// which may choose the second best shape, by as much.
 struct GemmShape {
   int mt, wn, wk;
   float turn_us;

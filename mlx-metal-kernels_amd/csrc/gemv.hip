@@ -6,11 +6,20 @@
 // q4 codes are packed two per byte (low nibble = even k), so on little-endian
 // hardware a 32-bit word holds 8 consecutive codes, nibble i at bits 4i.
 //
-// 33 and more rows take the product kernel (gemm.hip).  Decode batches of at
-// most 4 rows (q8: 2) with fp16 activations and scales take the v_dot2 kernel
-// below, 17-32 rows the two-column-tile kernel; the rest, bf16 and fp32
-// scales the MFMA path:
-// Fast path (M <= 16 per launch, K % 64 == 0 for q4 / % 32 for q8, power-of-two
+// Who takes a launch (gemv_dispatch; each kernel's own conditions stand at its
+// *_eligible or *_ok function):
+//   1-4 rows (q8: 2), fp16 with fp16 scales, also those that passes of 32 leave
+//     over: the v_dot2 kernel below;
+//   up to 32 rows (q8: 16), fp16 scales, any activation type: the few-row kernel
+//     (gemv_few.hip), in two passes up to twice that; without a workspace rows of
+//     up to 4096 k only;
+//   33 and more rows (q8 pairs and fp16: 17): the product kernel (gemm.hip), or
+//     two passes where that is faster;
+//   fp16 with fp16 scales, where they are faster or the few-row kernel does not
+//     apply: the K-split kernel (one q4 matrix) and the tile kernel (17-32 rows);
+//   what is left, fp32 scales above all: the MFMA kernel of 16 rows a launch, and
+//     the generic kernel for odd layouts.
+// The MFMA kernel (M <= 16 per launch, K % 64 == 0 for q4 / % 32 for q8, power-of-two
 // group size >= 16 (q4) / >= 8 (q8)):
 //   * one workgroup owns a 16-row output tile; its KW waves split K;
 //   * lane (n = l%16, kb = l/16) streams 32 contiguous code bytes of row n per
@@ -194,8 +203,9 @@ __global__ __launch_bounds__(512) void gemv_mfma_kernel(const GemvArgs args) {
 // --------------------------------------------------------------------------
 // Batched decode tile kernel: fp16 activations and fp16 scales, M <= 16 * MT
 // rows per launch, power-of-two group size >= 32, K % 128 == 0.  Used with
-// MT = 2 for 17-32 rows (a batch-32 decode step): one pass over the weights
-// instead of two 16-row MFMA passes.
+// MT = 2 for 17-32 rows that the few-row and product kernels do not take or take
+// longer for (tile_rows_us): one pass over the weights instead of two 16-row
+// MFMA passes.
 //
 // A workgroup owns 16 output rows of NMAT matrices; its kw waves split K
 // into 128-k chunks.  Per chunk, lane (r = l % 16, kb = l / 16) takes the 32
@@ -369,10 +379,12 @@ __global__ __launch_bounds__(NMAT == 1 && BITS == 4 ? 1024 : 512) void gemv_tile
 
 // --------------------------------------------------------------------------
 // K-split batched kernel (q4, fp16 activations and scales, 5..32 rows, one
-// matrix, K % 128 == 0 with 2048 <= K <= 16384, N % 16 == 0): long rows (the
-// 14336-k down projection) of calls that give no workspace, which the few-row
-// kernel needs to split them over workgroups.  One 16-row tile per workgroup of 16 waves; wave w takes an
-// equal run of the row's 128-k halves (7 at K = 14336) and requests all of its
+// matrix, K % 128 == 0 with 2048 <= K <= 16384, N % 16 == 0): long rows, in one
+// launch where the few-row kernel cuts them into slices and sums those through a
+// workspace -- of calls that give none, and of the batch sizes that one round of
+// it takes sooner (gemv_dispatch).  One 16-row tile per workgroup of 16 waves;
+// wave w takes an equal run of the row's 128-k halves (7 at K = 14336) and
+// requests all of its
 // codes up front (one 16-byte load per half: lane (r, kb) reads k in
 // [128 h + 32 kb, +32) of row r, so each instruction reads the 16 rows'
 // aligned 64-byte half lines), then walks its halves with the activations of
@@ -1074,12 +1086,11 @@ int launch_fast(const GemvArgs& a, int gpc, hipStream_t st) {
   return MK_OK;
 }
 
-// Tile kernel plan: ring depth NB (4 chunks for q4 at one column tile; 2
-// where the x or q8 code registers double) and kw waves per 16-row tile,
-// kw <= 16 for a single q4 matrix, else 8 (1024 / 512 threads), preferring a
-// split that gives every wave a whole number of rings and at least one.
-template <int BITS, int MT>
-constexpr int tile_ring() { return BITS == 4 && MT == 1 ? 4 : 2; }
+// Tile kernel plan: rings of two chunks (the registers that two column tiles'
+// activations leave) and kw waves per 16-row tile, kw <= 16 for a single q4
+// matrix, else 8 (1024 / 512 threads), preferring a split that gives every wave a
+// whole number of rings and at least one.
+constexpr int kTileRing = 2;
 
 template <int BITS, int NMAT>
 inline int tile_choose_kw(int64_t K, int nb) {
@@ -1093,7 +1104,7 @@ inline int tile_choose_kw(int64_t K, int nb) {
 
 template <int BITS, int NMAT, int MT, int EPI>
 int launch_tile(GemvArgs a, hipStream_t st) {
-  constexpr int NB = tile_ring<BITS, MT>();
+  constexpr int NB = kTileRing;
   a.kw = tile_choose_kw<BITS, NMAT>(a.K, NB);
   if (a.kw < MT) a.kw = MT;  // wave j finishes column tile j
   const dim3 grid((unsigned)((a.N + 15) / 16));
@@ -1414,8 +1425,8 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
     }
   }
   int64_t m_done = 0;
-  // up to 32 rows at a time through the K-split kernel (long rows without a
-  // workspace)
+  // up to 32 rows at a time through the K-split kernel (ksplit, and long rows
+  // without a workspace)
   if constexpr (NMAT == 1) {
     if (M - m_done >= kXkMinRows && xk_eligible<BITS, NMAT>(a, 1, act_dt, sc_dt)) {
       while (M - m_done >= kXkMinRows && rc == MK_OK) {
@@ -1694,7 +1705,8 @@ int norm_qkv_rope_entry(const void* x, const void* norm_w, float eps, const uint
     bool fast;
     gemv_prepare<BITS, 1>(probe, N, K, gs, &fast);
     // from kGemmMinRows rows on, one product of all rows and the update kernel
-    // beat passes of 32 rows with the update in their epilogue (same bytes)
+    // beat passes of 32 rows with the update in their epilogue (the same arithmetic,
+    // fp32 sums in another order)
     const bool product = M >= kGemmMinRows && gemm_rows_ok<BITS, 1>(probe, M, gs);
     if (fast && !product) {
       int rc = mk_rms_norm(x, norm_w, normed_out, M, K, eps, act_dt, nw_dt, stream);

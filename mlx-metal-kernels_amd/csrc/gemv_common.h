@@ -55,7 +55,8 @@ __device__ __forceinline__ u32x4 xperm(u32x4 X) {
 // exactly in fp16 for |zi| < 1024 -- so w = fma(c - zi, s, corr) with
 // corr = -(z - zi) s rounds once, to the fp16 of (c - z) s whenever z is an
 // integer (the rounding of the reference's fp32 dequant, for any fp16 scale),
-// and keeps a fractional z exact to ulp(corr).
+// and keeps a fractional z exact to ulp(corr).  (Zero points past 1024 lose bits
+// of 1024 + zi; the layouts of gemv_generic_kernel never come here.)
 struct GpMagic {
   f16x2 s;     // (s, s)
   f16x2 kz;    // (1024 + zi)
@@ -172,11 +173,6 @@ template <>
 __device__ __forceinline__ f32x4 mfma_k32<bf16>(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8>(a), bitcast<bf16x8>(b), c, 0, 0,
                                                  0);
-}
-
-template <typename ST>
-__device__ __forceinline__ float ld_scalar_f32(const ST* p) {
-  return to_f32(*p);
 }
 
 // The decode token's cache write fused into the qkv projection's epilogue
@@ -486,8 +482,8 @@ template <int BITS, int NMAT, int EPI>
 int launch_gemm_rows(const GemvArgs& a, int act_dt, int sc_dt, hipStream_t st);
 
 // The few-row matvec (gemv_few.hip), a.M <= 32 rows (8-bit codes: 16) of what
-// few_ok accepts, with few_workspace_bytes of workspace (0 unless K is cut into
-// slices; EPI_ROPE_KV and EPI_GATE_UP need it 0).
+// few_ok accepts, with few_workspace_bytes of workspace (0 unless K > 4096 is cut
+// into slices; EPI_ROPE_KV and EPI_GATE_UP need it 0, so their K ends at 4096).
 size_t few_workspace_bytes(int64_t M, int64_t N, int64_t K);
 template <int BITS, int NMAT>
 bool few_ok(const GemvArgs& a, int64_t M, int64_t gs, int sc_dt, size_t ws_bytes);
