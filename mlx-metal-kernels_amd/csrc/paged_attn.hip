@@ -250,10 +250,10 @@ __device__ __forceinline__ u32x4 deq4x8(uint32_t u, f16x2 s2, Q4Magic mg) {
 // consumed.  Loads are branch-free -- positions past the split's end or on
 // an unmapped page read a clamped in-bounds row and are masked out of the
 // softmax (their V is zeroed) -- so the compiler's wait counts stay exact.
-// Quantized caches are bound by the vector ALU (q4: 75 % of its cycles issue),
+// Quantized caches are bound by the vector ALU (q4: it issues in 59 % of cycles),
 // so what every lane would compute alike is kept in scalar registers: the wave
 // index and a pair's block count are made scalar, and with them page rows,
-// bases and branches.  Per block and wave 531 -> about 400 vector instructions
+// bases and branches.  Per block and wave 531 -> 406 vector instructions
 // with q4's and-or unpacking, us per call (32 / 8 heads of 128): q4 8 x 32768
 // positions 94.4 -> 80.4, 32 x 8192 76.8 -> 64.2; q8 8 x 32768 116 -> 109; fp16
 // (bound by the pages' stream) unchanged.  A third block buffer for q4, 2 blocks
