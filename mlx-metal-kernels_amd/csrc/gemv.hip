@@ -1327,7 +1327,7 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
     if (M > pass && dot_eligible<BITS, NMAT>(a, fast, tail, act_dt, sc_dt)) {
       // us at 33 / 36 / 65 rows, all rows in one form -> this, q4 g64:
       // 2 x 14336 x 4096 36 / 35 / 53 -> 35 / 42 / 47, 6144 x 4096 18 / 18 / 22
-      // -> 16 / 18 / 26, 4096 x 14336 35 / 36 / 67 -> 28 / 32 / 48
+      // -> 16 / 18 / 26, 4096 x 14336 35 / 36 / 67 -> 24 / 28 / 41
       rc = gemv_dispatch<BITS, NMAT, EPI>(a, M - tail, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes, BITS == 4 && NMAT == 2 ? 32 : 33);
       if (rc != MK_OK) return rc;
       GemvArgs b = a;
