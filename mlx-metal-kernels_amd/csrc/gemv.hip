@@ -1276,10 +1276,11 @@ inline float tile_rows_us(int64_t M, int64_t N, int64_t K) {
   return 3.0f + rounds * us * rows * (float)K / 1024.0f;
 }
 
-// Rows of a whole pass: the 1-4 rows (q8: 2) that a batch leaves past its last
-// one take the v_dot2 kernel, which does not round W, as when every batch ran in
-// passes.  (16 where two column tiles' partial sums and a pair's 128 groups of
-// 32 did not fit LDS together.)
+// Rows of a whole pass.  The 1-4 rows (q8: 1-2) that a batch leaves past its last
+// one take the v_dot2 kernel, which does not round W: other kernels would hold
+// their weights in fp16 only because of the rows beside them (error of such a row
+// against 64 bits 2.1e-4, 3.0e-4 with rounded weights).  32 rows, or 16: where the
+// tile kernel does not apply, and for pairs of 128 groups of 32.
 template <int BITS, int NMAT>
 inline int64_t pass_rows(int64_t N, int64_t K, int64_t gs) {
   const bool pair32 = BITS == 4 && NMAT == 2 && K == 4096 && gs == 32 && N % 16 == 0 && N >= 4096;
@@ -1328,7 +1329,8 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
       // us at 33 / 36 / 65 rows, all rows in one form -> this, q4 g64:
       // 2 x 14336 x 4096 36 / 35 / 53 -> 35 / 42 / 47, 6144 x 4096 18 / 18 / 22
       // -> 16 / 18 / 26, 4096 x 14336 35 / 36 / 67 -> 24 / 28 / 41
-      rc = gemv_dispatch<BITS, NMAT, EPI>(a, M - tail, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes, BITS == 4 && NMAT == 2 ? 32 : 33);
+      rc = gemv_dispatch<BITS, NMAT, EPI>(a, M - tail, N, K, gs, act_dt, sc_dt, st, ws, ws_bytes,
+                                          BITS == 4 && NMAT == 2 ? 32 : kGemmMinRows);
       if (rc != MK_OK) return rc;
       GemvArgs b = a;
       b.M = (int)tail;
@@ -1373,7 +1375,8 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
     // against 4.6, q8 fp16 at 8 rows 3.3 against 4.0, q8 bf16 at 32 rows 6.6 against
     // 8.6; 2 x 2048 x 512 q4 fp16 at 17 rows 4.3 against 6.3; 2 x 8192 x 512 bf16 6.9
     // against 6.0; 2 x 4864 x 896 at 17 rows 7.2 against 8.9)
-    const bool brief = fast && ((K <= 512 && tiles <= 128 && (BITS == 8 || act_dt == MK_DT_F16 ? M <= 32 : M <= 16)) ||
+    const int64_t few_rows = BITS == 8 || act_dt == MK_DT_F16 ? 32 : 16;
+    const bool brief = fast && ((K <= 512 && tiles <= 128 && M <= few_rows) ||
                                 (NMAT == 2 && K < 1024 && K % 512 != 0 && M >= 17 && M <= 32 &&
                                  tile_eligible<NMAT>(a, act_dt, sc_dt)));
     const bool few = M <= 2 * kPass && !ksplit && !uneven && !brief && !dot_eligible<BITS, NMAT>(a, fast, M, act_dt, sc_dt) &&
@@ -1383,7 +1386,8 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
     const bool few_rest = M > 32 && M <= 48 && few_ok<BITS, NMAT>(a, M - 32, gs, sc_dt, ws_bytes);
     if constexpr (EPI != EPI_ROPE_KV) {
       const bool tile = tile_eligible<NMAT>(a, act_dt, sc_dt);
-      bool product = (M >= product_rows || (wide8 && (NMAT == 2 || tile))) && M < (1LL << 24) && gemm_rows_ok<BITS, NMAT>(a, M, gs);
+      bool product = (M >= product_rows || (wide8 && (NMAT == 2 || tile))) && M < (1LL << 24) &&
+                     gemm_rows_ok<BITS, NMAT>(a, M, gs);
       if (product && M < kGemmMinRows && tile && !(BITS == 4 && few)) {
         // (short rows: the estimate leaves out what every workgroup takes to start)
         const float us = (K <= 1024 ? 1.25f : 0.9f) * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K);

@@ -43,7 +43,8 @@ def test_few_rows(dev, M, N, K, bits, dtype):
 @pytest.mark.parametrize("g", [32, 64, 128, 256])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("M,N,K", [(5, 7, 64), (8, 300, 1024), (12, 14336, 512), (32, 9000, 1024), (24, 100, 4096), (16, 3000, 1056)])
+@pytest.mark.parametrize("M,N,K", [(5, 7, 64), (8, 300, 1024), (12, 14336, 512), (32, 9000, 1024), (24, 100, 4096),
+                                   (16, 3000, 1056)])
 def test_few_rows_gate_up(dev, M, N, K, bits, dtype, g):
     gen = torch.Generator(device=dev).manual_seed(M + N + K)
     x = torch.randn((M, K), generator=gen, device=dev).to(dtype)
@@ -66,7 +67,8 @@ def test_few_rows_bf16_small(dev, M):
         x = torch.randn((M, K), generator=gen, device=dev).bfloat16()
         codes, packed, s, z = _weight(gen, dev, N, K, bits, 32, torch.float16, "whole")
         fn = qo.q4_matvec_decode if bits == 4 else qo.q8_matvec_decode
-        _check(fn(x, packed, s, z, group_size=32), x, _rounded(codes, s, z, 32, torch.bfloat16), torch.bfloat16, (M, N, K))
+        _check(fn(x, packed, s, z, group_size=32), x, _rounded(codes, s, z, 32, torch.bfloat16), torch.bfloat16,
+               (M, N, K))
 
 
 @pytest.mark.parametrize("bits", [4, 8])
@@ -88,7 +90,8 @@ def test_few_rows_unaligned_scales_and_no_workspace(dev, bits):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("M,K,g", [(6, 96, 32), (16, 544, 64), (8, 1056, 128), (16, 4608, 32), (7, 4608, 64), (5, 4608, 128)])
+@pytest.mark.parametrize("M,K,g", [(6, 96, 32), (16, 544, 64), (8, 1056, 128), (16, 4608, 32), (7, 4608, 64),
+                                   (5, 4608, 128)])
 def test_few_rows_infinite_weights_before_k_ends(dev, M, K, g, bits):
     """Rows whose first weights are infinite in fp16 give the saturated sum, also
     where blocks (or whole waves) past K re-read them against zero activations."""

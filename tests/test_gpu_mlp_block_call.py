@@ -1,7 +1,7 @@
 """The MLP block in one library call against its two calls (norm + gate/up,
 then down + residual): the same kernels on the same values, so the outputs are equal
 bit for bit.  One row to
-more than the workspace's 64, both weight types, hidden sizes with and without
+more than the workspace's 68, both weight types, hidden sizes with and without
 a workspace for the down projection, inputs that are views."""
 
 import pytest
@@ -29,6 +29,7 @@ def _linear(g, bits, n, k, gs, scale_dtype, zeros):
     ((2, 16, 256), 8192, 8, 128, torch.float16, torch.float16, False),
     ((64, 1, 128), 4128, 4, 32, torch.float16, torch.float32, True),
     ((5, 13, 256), 512, 4, 32, torch.float16, torch.float16, True),
+    ((66, 1, 128), 8192, 4, 64, torch.float16, torch.float16, True),  # two rows past the last pass, K slices
     ((3, 1, 33), 65, 4, 32, torch.float16, torch.float16, True),  # odd sizes
 ])
 def test_block_equals_its_two_calls(shape, hidden, bits, gs, dtype, scale_dtype, zeros):
