@@ -46,13 +46,14 @@ def values_only(*tensors: torch.Tensor) -> bool:
     """Whether a kernel that reads the tensors' memory does all that tensor ops
     would: no gradient to record, no forward-mode tangent, no function transform
     (vmap, jvp, grad), no tracing, dispatch mode or tensor subclass."""
-    if (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+    if (torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None):  # (there even new tensors are wrapped)
         return False
+    grad, dual = torch.is_grad_enabled(), forward_ad._current_level >= 0
     for t in tensors:
-        if type(t) not in (torch.Tensor, torch.nn.Parameter):
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
             return False
-        if (t.requires_grad and torch.is_grad_enabled()) or forward_ad.unpack_dual(t).tangent is not None:
+        if (grad and t.requires_grad) or (dual and forward_ad.unpack_dual(t).tangent is not None):
             return False
     return True
 

@@ -224,34 +224,34 @@ def _hip_quantize_rows(pages: torch.Tensor, group_size: int, bits: int):
     if pages.dtype not in (torch.float16, torch.bfloat16):
         pages = pages.to(torch.float16)
     src = pages.contiguous()
-    dev = _lib.require_device(src)
+    dev = src.device if src.is_cuda else _lib.require_device(src)
     *lead, D = src.shape
     rows = src.numel() // D
-    G = (D + group_size - 1) // group_size
-    codes = torch.empty(tuple(lead) + ((D if bits == 8 else (D + 1) // 2),), dtype=torch.uint8, device=dev)
-    scales = torch.empty(tuple(lead) + (G,), dtype=torch.float16, device=dev)
-    _lib.launch("mk_quantize_kv", dev, _lib.ptr(src), _lib.ptr(codes), _lib.ptr(scales), rows, D, group_size, bits,
-                _lib.dtype_code(src.dtype))
+    codes = torch.empty((*lead, D if bits == 8 else (D + 1) // 2), dtype=torch.uint8, device=dev)
+    scales = torch.empty((*lead, (D + group_size - 1) // group_size), dtype=torch.float16, device=dev)
+    _lib.launch("mk_quantize_kv", dev, src.data_ptr(), codes.data_ptr(), scales.data_ptr(), rows, D, group_size, bits,
+                _lib.DT_F16 if src.dtype is torch.float16 else _lib.DT_BF16)
     return codes, scales
 
 
 def _hip_dequantize(codes: torch.Tensor, scales: torch.Tensor, group_size: int, bits: int, D: int):
     """mk_dequantize_kv of device codes [..., D | ceil(D/2)] with fp16 scales
     [..., ceil(D/group_size)] -> fp16 [..., D]; None for what the kernel does
-    not take (host tensors, other types or layouts, gradients, function
-    transforms and tracing), which stays with the tensor ops."""
-    want = tuple(codes.shape[:-1])
-    if (codes.device.type != "cuda" or scales.device != codes.device or codes.dtype != torch.uint8
-            or scales.dtype != torch.float16 or not values_only(codes, scales) or D <= 0
-            or group_size <= 0 or tuple(codes.shape) != want + (D if bits == 8 else (D + 1) // 2,)
-            or tuple(scales.shape) != want + ((D + group_size - 1) // group_size,)):
+    not take (host tensors, other types or layouts), which stays with the tensor
+    ops, as does what values_only says no to."""
+    shape = tuple(codes.shape)
+    lead = shape[:-1]
+    if (not codes.is_cuda or scales.get_device() != codes.get_device() or codes.dtype is not torch.uint8
+            or scales.dtype is not torch.float16 or D <= 0 or group_size <= 0
+            or shape != (*lead, D if bits == 8 else (D + 1) // 2)
+            or tuple(scales.shape) != (*lead, (D + group_size - 1) // group_size)):
         return None
-    codes, scales = codes.contiguous(), scales.contiguous()
-    out = torch.empty(want + (D,), dtype=torch.float16, device=codes.device)
-    if out.numel() == 0:
-        return out
-    _lib.launch("mk_dequantize_kv", codes.device, _lib.ptr(codes), _lib.ptr(scales), _lib.ptr(out), out.numel() // D, D,
-                group_size, bits)
+    codes, scales, dev = codes.contiguous(), scales.contiguous(), codes.device
+    out = torch.empty((*lead, D), dtype=torch.float16, device=dev)
+    n = out.numel()
+    if n:
+        _lib.launch("mk_dequantize_kv", dev, codes.data_ptr(), scales.data_ptr(), out.data_ptr(), n // D, D, group_size,
+                    bits)
     return out
 
 
@@ -276,6 +276,7 @@ def _dequantize_pages(paged_qkv: PagedQuantizedKVCache, kernel: bool):
     if orig is None:
         raise ValueError("original_page_shape is required for dequantization")
     D = orig[3]
+    kernel = kernel and values_only(paged_qkv.k_pages_q, paged_qkv.k_scales, paged_qkv.v_pages_q, paged_qkv.v_scales)
 
     def values(which, codes, scales):
         out = _hip_dequantize(codes, scales, paged_qkv.group_size, paged_qkv.bits, D) if kernel else None

@@ -25,7 +25,7 @@ from typing import Any
 import torch
 
 from . import _contig, _lib
-from ._common import ci_safe_mode_enabled
+from ._common import ci_safe_mode_enabled, values_only
 from .gqa_ops import validate_gqa_heads
 from .kv_cache_ops import normalize_positions
 from .paged_kv_ops import _masked_attention
@@ -177,6 +177,7 @@ def _dequantize_cache(qkv_cache: QuantizedKVCache, kernel: bool):
     qkv_cache = qkv_cache.validate()
     B, S, H, D = _geometry(qkv_cache)
     g, bits = qkv_cache.group_size, qkv_cache.bits
+    kernel = kernel and values_only(qkv_cache.k_q, qkv_cache.k_scales, qkv_cache.v_q, qkv_cache.v_scales)
 
     def values(which, codes, scales):
         out = _hip_dequantize(codes, scales, g, bits, D) if kernel else None
