@@ -1389,8 +1389,13 @@ int gemv_dispatch(GemvArgs a, int64_t M, int64_t N, int64_t K, int64_t gs, int a
       bool product = (M >= product_rows || (wide8 && (NMAT == 2 || tile))) && M < (1LL << 24) &&
                      gemm_rows_ok<BITS, NMAT>(a, M, gs);
       if (product && M < kGemmMinRows && tile && !(BITS == 4 && few)) {
-        // (short rows: the estimate leaves out what every workgroup takes to start)
-        const float us = (K <= 1024 ? 1.25f : 0.9f) * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K);
+        // (short rows: the estimate leaves out what a second round of workgroups
+        // takes to start.  Product and tile kernel, us at 32 rows: 2 x 20480 x 1024
+        // 24.1 and 22.8, 2 x 10400 x 1024 12.7 and 15.0, 2 x 5632 x 1024 9.6 and
+        // 10.9, 2 x 14336 x 512 9.5 and 10.0, at 17 rows 9.5 and 8.7)
+        const bool rounds = NMAT * N > 128 * cus;
+        const float by = K > 1024 ? 0.9f : rounds ? 1.2f : K <= 512 ? 1.05f : 0.95f;
+        const float us = by * gemm_rows_us(BITS, NMAT, (int)M, a.N, a.K);
         product = us < tile_rows_us<BITS, NMAT>(M, N, K);
       } else if (product && few && M <= kPass) {
         product = false;  // one pass
